@@ -1411,7 +1411,7 @@ struct Runner {
             q.in_max_len = o.din->l;
             q.in_start = o.din->wstart_d.as<int64_t>(), q.in_len = o.din->wlen_d.as<int64_t>();
         }
-        q.tiles = t.dev();
+        q.tiles = t.dev(), q.tile_wn = wn;
         if (o.t_hi >= 0) {  // a range of the tiles (they are in item order): a group of items
             q.tiles.item += o.t_lo, q.tiles.t0 += o.t_lo, q.tiles.n += o.t_lo;
             q.tiles.count = o.t_hi - o.t_lo;

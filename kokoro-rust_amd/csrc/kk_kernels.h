@@ -88,6 +88,7 @@ struct ConvParams {
     const int64_t* out_start;// ConvT: output domain item spans
     const int64_t* out_len;
     StatPart* part;          // epilogue statistics [tiles * WN][cout] (null: none)
+    int tile_wn;             // 128-column spans per tile (the tile width / 128: WN)
 };
 
 // in_h / out_h: fp16 input (conv2 of a Snake step) / fp16 output (conv1 of a Snake step).
@@ -95,6 +96,24 @@ struct ConvParams {
 // against the kernel's limits (hipErrorInvalidValue when out of range) and launch nothing.
 hipError_t launch_conv(const ConvParams& p, int pro, int epi, int shape, bool stats, bool in_h, bool out_h, int n_cu,
                        hipStream_t s, bool validate_only = false);
+
+// The narrow kernel (kk_conv_narrow.hip): up to kConvGroup layers of one (prologue, epilogue, ...)
+// combination in one launch, each block a part of the 64-row x 128-column units of one layer;
+// first[] is filled in.
+constexpr int kConvGroup = 3;
+struct ConvGroup {
+    ConvParams p[kConvGroup];
+    int first[kConvGroup];  // the first block of each layer
+    int n;
+};
+hipError_t launch_conv_narrow(ConvGroup& g, int pro, int epi, bool stats, bool in_h, bool out_h, hipStream_t s);
+// launch_conv runs a layer there when its 64 x 128 units are at most one per CU (256).  Measured
+// per layer and call: a 40-frame item's decoder conv1 (16 units) 38 -> 20 us, its Snake convs (28
+// and 76 units) 21-34 -> 9-16 us, a 112-row linear of 768 channels (12 units) 16 -> 9 us; calls whose
+// layers lie between 256 and 512 units (a 676-frame item's stage 0) got 3% slower with the line at
+// 512, and batches of 1,200 frames 10% at 1,024.
+constexpr int64_t kNarrowUnits = 256;
+inline int64_t conv_units64(const ConvParams& p) { return p.tiles.count * p.tile_wn * (p.m_pad / 64); }
 
 // ---------------------------------------------------------------- bandwidth kernels (kk_misc.hip)
 // Statistics partials of x [l][ld] over tiles (one partial per tile and channel).
