@@ -772,7 +772,7 @@ struct kk_plan {
         }
         return *it->second;
     }
-    // the quad recurrences' schedule over the items of domain d (built on first use, like the tiles)
+    // the grouped recurrences' schedule over the items of domain d (built on first use, like the tiles)
     std::map<const kk::Dom*, kk::DevBuf> lstm_sched;
     const int32_t* lstm_sched_of(const kk::Dom& d) {
         auto it = lstm_sched.find(&d);
@@ -796,10 +796,11 @@ struct kk_plan {
     kk::DevBuf ids, row_item, att_item, att_head, att_q0, style_pro, gbp;
     kk::DevBuf u_emb, u_h, u_qkv, u_ctx, u_ffn, u_x, u_gx, u_xl, u_logits, u_te, u_te2, u_gxt, u_gxs, u_sh;
     kk::DevBuf u_fx[2], u_fpool[2], u_fh[2], u_fsc[2], u_fy[2];  // the F0 and N stacks
-    // the two-CU recurrences' exchange words: word 0 the run's abort flag, then one region per
-    // stream that runs recurrences (the main stream, and side stream 0 for the text encoder)
+    // the recurrences' exchange words: word 0 the run's abort flag, then a region for each of a run's
+    // recurrences (text encoder, three duration encoder, duration, shared)
     kk::DevBuf u_lstmx;
-    static constexpr int64_t kLstmXHead = 64;
+    static constexpr int64_t kLstmXHead = 64, kLstmRegions = 6;
+    static int64_t lstm_words(int n) { return kLstmXHead + kLstmRegions * 2 * (int64_t)n * 512; }
     int64_t n_att = 0;
     float* logits_host = nullptr;  // pinned, grow-only (the duration logits come back through it)
     size_t logits_cap = 0;
@@ -1817,24 +1818,25 @@ struct Runner {
     }
     // BiLSTM recurrence over the item spans of d (gx rows through gx_row, or the spans' own rows);
     // h into out[row][0:512].  Algorithmic traffic: gx read and h written once per row, W_hh once.
-    // Each sequence runs on four CUs (launch_lstm_quad, at most 64 quads running scheduled lists)
-    // when the longest span has at least kLstmQuadMinSteps steps (below, the quads' per-step gain
-    // does not pay for their lists), else on two (launch_lstm_pair; bit-identical), with its
-    // exchange words in `region` (one per stream that runs recurrences at the same time);
-    // KOKORO_HIP_LSTM_SINGLE=1 selects the one-CU kernel (W_hh partly streamed from L2 each step),
-    // as does a plan whose pairs or quads gave up before (lstm_single).  Test hook, read at each
-    // launch: KOKORO_HIP_TEST_LSTM_SILENT=1 keeps the second half of every pair (the second quarter
-    // of every quad) from publishing and cuts the wait to 10 us, so that they give up.
+    // Each sequence runs on 16, 8 or 4 CUs (launch_lstm_split; lstm_parts: as many as 256 CUs hold for
+    // every sequence at once) when all the sequences run at once, and on groups of 4 with scheduled
+    // lists when the longest span has at least kLstmQuadMinSteps steps; else on two (launch_lstm_pair;
+    // bit-identical).  `region`: the launch's exchange words, its own within a run (tokens() clears
+    // them all).  KOKORO_HIP_LSTM_SINGLE=1 selects the one-CU kernel (W_hh partly streamed from L2
+    // each step), as does a plan whose pairs or groups gave up before (lstm_single).  Test hook, read
+    // at each launch: KOKORO_HIP_TEST_LSTM_SILENT=1 keeps the second half of every pair (the second
+    // part of every group) from publishing and cuts the wait to 10 us, so that they give up.
+    //   Measured per step: 2.0 us on two CUs, see lstm_split_kernel for the others.
     void recur(const MLstm& l, const float* gx, const int32_t* gx_row, const Dom& d, float* out, int64_t out_ld,
-               const std::string& name, int region = 0) {
+               const std::string& name, int region) {
         static const bool single = env_i64("KOKORO_HIP_LSTM_SINGLE", 0) != 0;
-        // KOKORO_HIP_LSTM_QUAD, read at each launch: 1 quads, 0 pairs for every span
+        // KOKORO_HIP_LSTM_QUAD, read at each launch: 1 groups, 0 pairs for every span
         check((int)d.len.size() == p->nb, "internal: recurrence domain");
         const int32_t* sched = p->lstm_sched_of(d);
         int64_t longest = 0;
         for (int64_t v : d.len) longest = std::max(longest, v);
         const int64_t qsel = env_i64("KOKORO_HIP_LSTM_QUAD", -1);
-        const bool quad = qsel < 0 ? longest >= kLstmQuadMinSteps : qsel != 0;
+        const bool split = qsel < 0 ? 2 * p->nb <= kLstmGroups || longest >= kLstmQuadMinSteps : qsel != 0;
         const bool silent = env_i64("KOKORO_HIP_TEST_LSTM_SILENT", 0) != 0;
         const double v = (double)d.valid();
         label = name;
@@ -1843,14 +1845,14 @@ struct Runner {
                 return launch_lstm(gx, 2048, gx_row, d.start_d.as<int64_t>(), d.len_d.as<int64_t>(), p->nb,
                                    l.whh_t.as<float>(), l.bhh.as<float>(), out, out_ld, s);
             uint64_t* x = p->u_lstmx.as<uint64_t>();
-            if (quad)
-                return launch_lstm_quad(gx, 2048, gx_row, d.start_d.as<int64_t>(), d.len_d.as<int64_t>(), p->nb,
-                                        sched, l.whh_t.as<float>(), l.bhh.as<float>(), out, out_ld,
-                                        x + kk_plan::kLstmXHead + (int64_t)region * 2 * p->nb * 512, (int*)x, s,
-                                        silent ? 1000 : kLstmPairWaitTicks, silent ? 1 : -1);
+            uint64_t* words = x + kk_plan::kLstmXHead + (int64_t)region * 2 * p->nb * 512;
+            if (split)
+                return launch_lstm_split(lstm_parts(p->nb), gx, 2048, gx_row, d.start_d.as<int64_t>(),
+                                         d.len_d.as<int64_t>(), p->nb, sched, l.whh_t.as<float>(), l.bhh.as<float>(),
+                                         out, out_ld, words, (int*)x, s, silent ? 1000 : kLstmPairWaitTicks,
+                                         silent ? 1 : -1);
             return launch_lstm_pair(gx, 2048, gx_row, d.start_d.as<int64_t>(), d.len_d.as<int64_t>(), p->nb,
-                                    l.whh_t.as<float>(), l.bhh.as<float>(), out, out_ld,
-                                    x + kk_plan::kLstmXHead + (int64_t)region * 2 * p->nb * 512, (int*)x, s,
+                                    l.whh_t.as<float>(), l.bhh.as<float>(), out, out_ld, words, (int*)x, s,
                                     silent ? 1000 : kLstmPairWaitTicks, silent ? 1 : -1);
         });
     }
@@ -1884,7 +1886,7 @@ struct Runner {
             std::swap(in, out);
         }
         linear(u.te_lstm.wih, in, 512, p->dtf, p->u_gxt.as<float>(), 2048, "text_encoder.lstm.ih");
-        recur(u.te_lstm, p->u_gxt.as<float>(), nullptr, dt, p->t_en.as<float>(), 512, "text_encoder.lstm", 1);
+        recur(u.te_lstm, p->u_gxt.as<float>(), nullptr, dt, p->t_en.as<float>(), 512, "text_encoder.lstm", 0);
     }
     // The token phase (src/gpu_batch.rs:198-248): ALBERT, bert_encoder, the duration encoder, the
     // duration LSTM and projection (logits [rows][kLogitsLd]), the shared LSTM's gate
@@ -1898,7 +1900,9 @@ struct Runner {
         const double v = (double)dt.valid();
         const bool conc = !ctx->profiling && !dry;
         hipStream_t main_s = s;
-        if (!dry) KK_HIP(launch_clear_u64(p->u_lstmx.as<uint64_t>(), 1, s));  // the run's abort flag
+        // the run's abort flag and the exchange words of all of its recurrences (the shared LSTM's
+        // too: a run whose token phase ran at plan creation uses the words cleared then)
+        if (!dry) KK_HIP(launch_clear_u64(p->u_lstmx.as<uint64_t>(), kk_plan::lstm_words(p->nb), s));
         if (conc) {
             KK_HIP(hipEventRecord(p->te_ev[0], main_s));
             KK_HIP(hipStreamWaitEvent(ctx->side[0], p->te_ev[0], 0));
@@ -1958,12 +1962,12 @@ struct Runner {
         for (int i = 0; i < 3; i++) {
             const std::string nm = "predictor.text_encoder.lstms." + std::to_string(2 * i);
             linear(u.dur_lstm[i].wih, X, 640, dtf, GX, 2048, nm + ".ih");
-            recur(u.dur_lstm[i], GX, nullptr, dt, X, 640, nm);
+            recur(u.dur_lstm[i], GX, nullptr, dt, X, 640, nm, 1 + i);
             layernorm(X, 640, 512, nullptr, nullptr, u.dur_gb_off[i], 1e-5f, false,
                       "predictor.text_encoder.lstms." + std::to_string(2 * i + 1));
         }
         linear(u.pred_lstm.wih, X, 640, dtf, GX, 2048, "predictor.lstm.ih");
-        recur(u.pred_lstm, GX, nullptr, dt, p->u_xl.as<float>(), 512, "predictor.lstm");
+        recur(u.pred_lstm, GX, nullptr, dt, p->u_xl.as<float>(), 512, "predictor.lstm", 4);
         linear(u.dur_proj, p->u_xl.p, 512, dtf, p->u_logits.as<float>(), kLogitsLd, "predictor.duration_proj");
         // the shared LSTM's gate pre-activations on the token rows: a frame's are its token's
         linear(u.shared.wih, X, 640, dtf, p->u_gxs.as<float>(), 2048, "predictor.shared.ih");
@@ -2038,7 +2042,7 @@ struct Runner {
     // stream 0 beside F0 (each with its own statistics region and AdaIN coefficients).
     void prosody() {
         recur(m.up.shared, p->u_gxs.as<float>(), p->src_row.as<int32_t>(), p->dn, p->u_sh.as<float>(), 512,
-              "predictor.shared");
+              "predictor.shared", 5);
         pro_style = true;
         const bool conc = !ctx->profiling && !dry;
         hipStream_t main_s = s;
@@ -2225,7 +2229,7 @@ static void init_full_plan(kk_plan* p, const kk_item* items, int n) {
     alloc_buf(p, p->u_gxt, R * 2048 * sizeof(float));
     alloc_buf(p, p->u_gxs, R * 2048 * sizeof(float));
     alloc_buf(p, p->t_en, R * 512 * sizeof(float));
-    alloc_buf(p, p->u_lstmx, (size_t)(kk_plan::kLstmXHead + 2 * 2 * (int64_t)n * 512) * sizeof(uint64_t));
+    alloc_buf(p, p->u_lstmx, (size_t)kk_plan::lstm_words(n) * sizeof(uint64_t));
     if (!p->abort_host) KK_HIP(hipHostMalloc((void**)&p->abort_host, sizeof(uint64_t), hipHostMallocDefault));
     p->t_rows = rows;
     for (auto& e : p->te_ev)

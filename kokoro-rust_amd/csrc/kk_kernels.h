@@ -251,7 +251,7 @@ hipError_t launch_attention(const float* qkv, const int64_t* start, const int64_
 hipError_t launch_lstm(const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start, const int64_t* len,
                        int nb, const float* whh_t, const float* bhh, float* out, int64_t out_ld, hipStream_t s);
 // The same recurrence with each (item, direction) split over two CUs that trade their halves of h
-// every step (the whole of W_hh on chip).  xbuf: 2 nb x 512 exchange words (cleared by the launch);
+// every step (the whole of W_hh on chip).  xbuf: 2 nb x 512 exchange words, zero before the launch;
 // *abort is set, and every block ends, if a block waits more than wait_ticks (100 MHz clock) for
 // its partner.  silent_half >= 0 (a test hook) keeps that half of every pair from publishing.
 constexpr uint64_t kLstmPairWaitTicks = 200000000ull;  // 2 s
@@ -259,22 +259,24 @@ hipError_t launch_lstm_pair(const float* gx, int64_t gx_ld, const int32_t* gx_ro
                             const int64_t* len, int nb, const float* whh_t, const float* bhh, float* out, int64_t out_ld,
                             uint64_t* xbuf, int* abort, hipStream_t s, uint64_t wait_ticks = kLstmPairWaitTicks,
                             int silent_half = -1);
-// Four CUs per (item, direction), each with a quarter of h and all of its W_hh rows in registers;
-// the same arguments (xbuf 2 nb x 512 words), bit-identical outputs.  lstm_quads(nb) quads (one
-// block per CU) run the 2 nb sequences as lists, sched = lstm_schedule(len, nb): [nq + 1] offsets,
-// then the sequence ids (2 item + direction) of each quad's list.  silent_quarter >= 0 (a test
-// hook) keeps that quarter of every quad from publishing.
-constexpr int kLstmQuads = 64;               // 256 CUs
-constexpr int64_t kLstmQuadMinSteps = 1024;  // the engine's choice: quads when a span has this many steps
-inline int lstm_quads(int nb) { return 2 * nb < kLstmQuads ? 2 * nb : kLstmQuads; }
+// `parts` = 4, 8 or 16 CUs per (item, direction), each with its share of h and of the W_hh rows in
+// registers; the same arguments, bit-identical outputs.  lstm_groups(nb) groups of `parts` blocks (at
+// most 256 blocks, one per CU) run the 2 nb sequences as lists, sched = lstm_schedule(len, nb): [nq + 1] offsets, then
+// the sequence ids (2 item + direction) of each group's list.  silent_part >= 0 (a test hook) keeps
+// that part of every group from publishing.
+constexpr int kLstmGroups = 64;              // of 4 blocks: 256 CUs
+constexpr int64_t kLstmQuadMinSteps = 1024;  // past 64 sequences: groups when a span has this many steps, else pairs
+inline int lstm_groups(int nb) { return 2 * nb < kLstmGroups ? 2 * nb : kLstmGroups; }
+// The most CUs per sequence that 256 hold at once: the fewer sequences, the shorter a step.
+inline int lstm_parts(int nb) { return lstm_groups(nb) <= 16 ? 16 : lstm_groups(nb) <= 32 ? 8 : 4; }
 // Longest processing time first: the sequences by decreasing length (items by length, ties by
-// index, both directions in turn), each to the quad with the least total length so far (ties: the
-// lowest quad).
+// index, both directions in turn), each to the group with the least total length so far (ties: the
+// lowest group).
 std::vector<int32_t> lstm_schedule(const int64_t* len, int nb);
-hipError_t launch_lstm_quad(const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start,
-                            const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
-                            float* out, int64_t out_ld, uint64_t* xbuf, int* abort, hipStream_t s,
-                            uint64_t wait_ticks = kLstmPairWaitTicks, int silent_quarter = -1);
+hipError_t launch_lstm_split(int parts, const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start,
+                             const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
+                             float* out, int64_t out_ld, uint64_t* xbuf, int* abort, hipStream_t s,
+                             uint64_t wait_ticks = kLstmPairWaitTicks, int silent_part = -1);
 // Zeroes n 64-bit words.
 hipError_t launch_clear_u64(uint64_t* x, int64_t n, hipStream_t s);
 // F0_proj / N_proj: y[r] = b + w . x[r][0:c] (c = 256) on the rows with col[r] >= 0, 0 elsewhere.

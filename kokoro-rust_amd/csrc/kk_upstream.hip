@@ -471,8 +471,8 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_kernel(const float* gx, int
 // buffer: one 64-bit word per unit, (step + 1) << 32 | bits(h), written and polled with relaxed
 // device-scope atomics -- a word carries its own step, so no fence orders data and flag.  Two
 // parities of words per half: a block overwrites the words of step s at step s + 2 only after its
-// partner has used them (the partner's step s + 1 needed them).  The buffer starts at zero each
-// launch (lstm_exchange_clear_kernel), the first valid tag is 1.
+// partner has used them (the partner's step s + 1 needed them).  The words start at zero each run
+// (lstm_exchange_clear_kernel: every launch of a run has words of its own), the first valid tag is 1.
 // Pairing: block B = 16 grp + 8 hf + x is half hf of sequence 8 grp + x, so the two halves sit 8
 // apart (the same XCD under round-robin dispatch, and consecutive on it).  Every wait is bounded:
 // past wait_ticks of the 100 MHz clock (or once another block gave up) the block sets *abort and
@@ -587,106 +587,152 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_pair_kernel(const float* gx
     }
 }
 
-// The BiLSTM recurrence on FOUR CUs per (item, direction): block quarter qb owns the 64 hidden units
-// [64 qb, 64 qb + 64), i.e. 256 gate rows, and keeps all of their W_hh in registers (thread t: the
-// gate rows g 256 + 64 qb + 2 (c mod 32) + {0, 1} with g = c / 32, c = t mod 128, over the
-// k-quarter q = t / 128: 64 k x 2 rows = 128 floats), so a step reads no weights from LDS and each
-// CU does half the pair kernel's multiply-adds.  Each step the block computes its 64 units of h and
-// trades them with its three partners through the same self-tagged 64-bit words as the pair kernel
-// (one word per unit, two parities per quarter: a block rewrites step s's words at step s + 2 only
-// after every partner has finished step s + 1, hence has read them); threads 0..63 compute and
-// publish the block's units while threads 64..255 wait for the partners' 192.  Every row's dot
-// product is summed in the pair kernel's order (the k-quarter's 64 terms in sequence, then the four
-// quarters as ((q0 + q1) + (q2 + q3)) + b_hh): the outputs are bit-identical to it.
-// The quarters of a quad are blocks 8 apart (the same XCD under round-robin dispatch) and 32
-// consecutive blocks hold 8 complete quads; a launch has at most kLstmQuads quads (one block per
-// CU), and each quad runs a list of sequences one after another, from a schedule the host computes
-// at plan creation: longest first, each sequence to the quad with the least work so far -- the
-// longest start at once, and the short ones follow on the quads that finish first, with no second
-// wave of blocks waiting for CUs.  A quad reloads its W_hh rows only when the direction changes;
-// every sequence starts from h = c = 0 and has its own exchange words.  A block whose partners
-// are not resident yet waits for CUs that finishing quads release (nothing a quad waits for
-// depends on a later one).  Every wait is bounded as in the pair kernel.
-//   sched: [nq + 1] list offsets, then the sequence ids (2 item + direction) of the quads' lists.
-__global__ void __launch_bounds__(kLstmThreads) lstm_quad_kernel(const float* gx, int64_t gx_ld, const int32_t* gx_row,
-                                                                 const int64_t* start, const int64_t* len,
-                                                                 const int32_t* sched, int nq, const float* whh_t,
-                                                                 const float* bhh, float* out, int64_t out_ld,
-                                                                 uint64_t* xbuf, int* abort, uint64_t wait_ticks,
-                                                                 int silent_quarter) {
-    __shared__ float part[4][256];  // partial dot products per k-quarter, local rows g 64 + u
-    __shared__ float hs[kH];        // h of the previous step
+// The BiLSTM recurrence on P = 4, 8 or 16 CUs per (item, direction): block part pt owns the U = 256 / P
+// hidden units [U pt, U pt + U), i.e. 4 U gate rows, and keeps all of their W_hh in registers (each
+// thread RPT gate rows over one 64-long k-quarter).  Each step a block computes its U units of h and
+// trades them with its partners through the same self-tagged 64-bit words as the pair kernel (one
+// word per unit, two parities per part: a block rewrites step s's words at step s + 2 only after every
+// partner has finished step s + 1, hence has read them).  A step in three phases, a barrier after
+// each: the dot products (the four k-quarters' sums to LDS); the gates, wave g the gate g of the
+// block's units (one transcendental on the critical path where one wave took four in a row);
+// wave 0 the cell update and the publication, while waves 4-7 wait for the partners' 256 - U words.
+// The gate pre-activations are loaded a step ahead (through gx_row two dependent loads, ~1 us).
+// Every row's dot product is summed in the pair kernel's order (the k-quarter's 64 terms in sequence,
+// then the four quarters as ((q0 + q1) + (q2 + q3)) + b_hh): the outputs are bit-identical to it.
+//   What bounds a step: the multiply-adds (1024 / 512 / 256 cycles of a SIMD at P = 4 / 8 / 16), a
+//   word's way through the XCD's L2 (0.27 us measured between two blocks of one XCD, 0.37 across),
+//   two transcendental evaluations and three barriers.
+// The parts of a sequence are blocks 8 apart (the same XCD under round-robin dispatch) and 8 P
+// consecutive blocks hold 8 complete sequences; a launch has at most 256 blocks (one per CU), and
+// each group of P blocks runs a list of sequences one after another, from a schedule the host
+// computes at plan creation: longest first, each sequence to the group with the least work so far --
+// the longest start at once, and the short ones follow on the groups that finish first, with no
+// second wave of blocks waiting for CUs.  A group reloads its W_hh rows only when the direction
+// changes; every sequence starts from h = c = 0 and has its own exchange words.  A block whose
+// partners are not resident yet waits for CUs that finishing groups release (nothing a group waits
+// for depends on a later one).  Every wait is bounded as in the pair kernel.
+//   sched: [nq + 1] list offsets, then the sequence ids (2 item + direction) of the groups' lists.
+// acc += w[k + i][e] h[i] for i = 0 .. 15 in sequence, h[i] in lane i of each row of 16 lanes of h: one
+// v_fmac_f32 with a DPP operand each (the compiler makes a move and a multiply-add of it).  The s_nop
+// covers the two wait states between a VALU write of h and its DPP read.
+template <int RPT>
+__device__ __forceinline__ void fma16(float& acc, float h, const float (&w)[64][RPT], int k, int e) {
+#define KK_FM(i, op) "v_fmac_f32_dpp %0, %1, %" #op " row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" KK_FM(0, 2) KK_FM(1, 3) KK_FM(2, 4) KK_FM(3, 5) KK_FM(4, 6) KK_FM(5, 7) KK_FM(6, 8) KK_FM(7, 9)
+            KK_FM(8, 10) KK_FM(9, 11) KK_FM(10, 12) KK_FM(11, 13) KK_FM(12, 14) KK_FM(13, 15) KK_FM(14, 16) KK_FM(15, 17)
+        : "+v"(acc)
+        : "v"(h), "v"(w[k][e]), "v"(w[k + 1][e]), "v"(w[k + 2][e]), "v"(w[k + 3][e]), "v"(w[k + 4][e]), "v"(w[k + 5][e]),
+          "v"(w[k + 6][e]), "v"(w[k + 7][e]), "v"(w[k + 8][e]), "v"(w[k + 9][e]), "v"(w[k + 10][e]), "v"(w[k + 11][e]),
+          "v"(w[k + 12][e]), "v"(w[k + 13][e]), "v"(w[k + 14][e]), "v"(w[k + 15][e]));
+#undef KK_FM
+}
+template <int P>
+__global__ void __launch_bounds__(kLstmThreads) lstm_split_kernel(const float* gx, int64_t gx_ld, const int32_t* gx_row,
+                                                                  const int64_t* start, const int64_t* len,
+                                                                  const int32_t* sched, int nq, const float* whh_t,
+                                                                  const float* bhh, float* out, int64_t out_ld,
+                                                                  uint64_t* xbuf, int* abort, uint64_t wait_ticks,
+                                                                  int silent_part) {
+    constexpr int U = kH / P, R = 4 * U;      // this block's units and gate rows
+    constexpr int RPT = P == 4 ? 2 : 1;       // gate rows per thread
+    constexpr int NQT = R / RPT;              // threads per k-quarter
+    static_assert(4 * NQT <= kLstmThreads && kH - U <= kLstmThreads - 256, "thread roles");
+    __shared__ float part[4][R];  // partial dot products per k-quarter, local rows gate U + unit
+    __shared__ float act[4][U];   // the gates
+    __shared__ float gxs[4][U];   // the step's gate pre-activations
+    __shared__ __align__(16) float hs[kH];  // h of the previous step
     __shared__ int gave_up;
-    const int B = blockIdx.x, qb = (B >> 3) & 3;
-    const int quad = (B >> 5) * 8 + (B & 7);
-    if (quad >= nq) return;  // the quad's other quarters return too
-    const int t = threadIdx.x, q = t >> 7, c = t & 127;
+    const int B = blockIdx.x, pt = (B >> 3) & (P - 1);
+    const int grp = (B / (8 * P)) * 8 + (B & 7);
+    if (grp >= nq) return;  // the group's other parts return too
+    const int t = threadIdx.x, q = t / NQT, c = t % NQT;
+    const bool mac = t < 4 * NQT;
     if (t == 0) gave_up = 0;
-    const int g = c >> 5, u0 = 2 * (c & 31);  // this thread's rows: gate g, units u0, u0 + 1 of the quarter
-    // threads 64..255: the partner quarter and unit they wait for
-    const int tp = t - 64, pq = (qb + 1 + tp / 64) & 3, pu = tp & 63;
-    const float* hq = hs + 64 * q;
-    float2 wr[64];
+    const int r0 = RPT * c, g = r0 / U, u0 = r0 % U;  // this thread's first row: gate g, unit u0
+    // waves 0-3: the gate ga of unit ua (lanes past U idle)
+    const int ga = (t >> 6) & 3, ua = t & 63;
+    const bool gate_thread = t < 256 && ua < U, load_thread = t >= 256 && ua < U;
+    // threads 256 ..: the partner part and unit they wait for
+    const int tp = t - 256, pq = (pt + 1 + (tp > 0 ? tp : 0) / U) & (P - 1), pu = tp & (U - 1);
+    const bool poll = tp >= 0 && tp < kH - U;
+    const float* hq = hs + 64 * (q & 3);
+    float wr[64][RPT];
     int wdir = -1;
-    const int li_end = sched[quad + 1];
-    for (int li = sched[quad]; li < li_end; li++) {
+    const int li_end = sched[grp + 1];
+    for (int li = sched[grp]; li < li_end; li++) {
         const int seq = sched[nq + 1 + li];
         const int item = seq >> 1, dir = seq & 1;
         const int64_t s0 = start[item], n = len[item];
         if (dir != wdir) {
-            const float* W = whh_t + (int64_t)dir * kH * 4 * kH + g * kH + 64 * qb + u0;
+            const float* W = whh_t + (int64_t)dir * kH * 4 * kH + g * kH + U * pt + u0;
 #pragma unroll
-            for (int k = 0; k < 64; k++) wr[k] = *(const float2*)(W + (int64_t)(64 * q + k) * 4 * kH);
+            for (int k = 0; k < 64; k++)
+#pragma unroll
+                for (int e = 0; e < RPT; e++) wr[k][e] = W[(int64_t)(64 * (q & 3) + k) * 4 * kH + e];
             wdir = dir;
         }
-        float cst = 0.f, bh[4];
-        if (t < 64) {
-#pragma unroll
-            for (int gg = 0; gg < 4; gg++) bh[gg] = bhh[dir * 4 * kH + gg * kH + 64 * qb + t];
-        }
+        float cst = 0.f, bh = 0.f;
+        if (gate_thread) bh = bhh[dir * 4 * kH + ga * kH + U * pt + ua];
         if (t < kH) hs[t] = 0.f;  // every read of the previous sequence's h ended before its last barrier
+        uint64_t* xw = xbuf + (int64_t)seq * 512 + pt * 2 * U;  // [parity][U] this part's words
+        const uint64_t* xr = xbuf + (int64_t)seq * 512 + pq * 2 * U + pu;
+        // the gate pre-activations of the next step, by waves 4-7; their row another step ahead.  (Not
+        // by the waves of the cell update: a load's wait there waits for the published words' stores
+        // too, ~1,400 cycles a step.)
+        const float* gxc = gx + dir * 4 * kH + ga * kH + U * pt + (ua & (U - 1));
+        auto row_of = [&](int64_t s) { return s0 + (dir == 0 ? s : n - 1 - s); };
+        // (kept as the loaded 32-bit word: widened where it is loaded, the widening waits for the load)
+        auto gx_row_of = [&](int64_t s) {
+            const int64_t r = row_of(s < n ? s : n - 1);
+            return gx_row ? gx_row[r] : (int32_t)r;
+        };
+        int32_t row_nxt = 0;
+        if (load_thread && n > 0) {
+            gxs[ga][ua] = gxc[(int64_t)gx_row_of(0) * gx_ld];
+            row_nxt = gx_row_of(1);
+        }
         __syncthreads();
-        uint64_t* xw = xbuf + (int64_t)seq * 512 + qb * 128;  // [parity][64] this quarter's words
-        const uint64_t* xr = xbuf + (int64_t)seq * 512 + pq * 128 + pu;
         for (int64_t step = 0; step < n; step++) {
-            const int64_t row = s0 + (dir == 0 ? step : n - 1 - step);
-            float gxv[4];
-            if (t < 64) {
-                const int64_t grow = gx_row ? (int64_t)gx_row[row] : row;
-#pragma unroll
-                for (int gg = 0; gg < 4; gg++) gxv[gg] = gx[grow * gx_ld + dir * 4 * kH + gg * kH + 64 * qb + t];
+            float gx_nxt = 0.f;
+            if (load_thread) {
+                gx_nxt = gxc[(int64_t)row_nxt * gx_ld];
+                row_nxt = gx_row_of(step + 2);
             }
-            float2 acc = make_float2(0.f, 0.f);
+            if (mac) {
+                // The quarter's 64 h, 16 per register in every row of 16 lanes; a multiply-add takes its h
+                // from lane k mod 16 of the row (DPP row_newbcast).  (Read as broadcast float4 they cost
+                // the LDS 1 KB per wave and read, 1,070 to 1,370 cycles a step.)
+                float hr[4];
 #pragma unroll
-            for (int k = 0; k < 64; k += 4) {
-                const float4 h4 = *(const float4*)(hq + k);
-                const float hv[4] = {h4.x, h4.y, h4.z, h4.w};
+                for (int k = 0; k < 4; k++) hr[k] = hq[16 * k + (t & 15)];
+                float acc[RPT];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    acc.x = fmaf(wr[k + e].x, hv[e], acc.x);
-                    acc.y = fmaf(wr[k + e].y, hv[e], acc.y);
-                }
+                for (int e = 0; e < RPT; e++) acc[e] = 0.f;
+#pragma unroll
+                for (int k = 0; k < 64; k += 16)
+#pragma unroll
+                    for (int e = 0; e < RPT; e++) fma16(acc[e], hr[k / 16], wr, k, e);
+#pragma unroll
+                for (int e = 0; e < RPT; e++) part[q][r0 + e] = acc[e];
             }
-            *(float2*)(&part[q][g * 64 + u0]) = acc;
+            __syncthreads();
+            if (gate_thread) {
+                const int r = ga * U + ua;
+                const float z = gxs[ga][ua] + (((part[0][r] + part[1][r]) + (part[2][r] + part[3][r])) + bh);
+                act[ga][ua] = ga == 2 ? tanhf(z) : sigmoid(z);
+            }
             __syncthreads();
             const uint64_t tag = (uint64_t)(step + 1) << 32;
-            if (t < 64) {
-                float gate[4];
-#pragma unroll
-                for (int gg = 0; gg < 4; gg++) {
-                    const int r = gg * 64 + t;
-                    gate[gg] = gxv[gg] + (((part[0][r] + part[1][r]) + (part[2][r] + part[3][r])) + bh[gg]);
-                }
-                const float ig = sigmoid(gate[0]), fg = sigmoid(gate[1]), gg2 = tanhf(gate[2]), og = sigmoid(gate[3]);
-                cst = fg * cst + ig * gg2;
-                const float h = og * tanhf(cst);
-                if (qb != silent_quarter)
-                    __hip_atomic_store(xw + (step & 1) * 64 + t, tag | __float_as_uint(h), __ATOMIC_RELAXED,
+            if (t < U) {
+                cst = act[1][t] * cst + act[0][t] * act[2][t];
+                const float h = act[3][t] * tanhf(cst);
+                if (pt != silent_part)
+                    __hip_atomic_store(xw + (step & 1) * U + t, tag | __float_as_uint(h), __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
-                hs[64 * qb + t] = h;
-                out[row * out_ld + dir * kH + 64 * qb + t] = h;
-            } else if (t < 256) {
-                const uint64_t* src = xr + (step & 1) * 64;
+                hs[U * pt + t] = h;
+                out[row_of(step) * out_ld + dir * kH + U * pt + t] = h;
+            } else if (poll) {
+                const uint64_t* src = xr + (step & 1) * U;
                 const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
                 uint64_t w;
                 for (uint32_t spin = 1;; spin++) {
@@ -699,8 +745,9 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_quad_kernel(const float* gx
                         break;
                     }
                 }
-                hs[64 * pq + pu] = __uint_as_float((uint32_t)w);
+                hs[U * pq + pu] = __uint_as_float((uint32_t)w);
             }
+            if (load_thread) gxs[ga][ua] = gx_nxt;  // this step's were read before the last barrier
             __syncthreads();
             if (gave_up) {
                 if (t == 0) __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -710,7 +757,7 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_quad_kernel(const float* gx
     }
 }
 
-// Zeroes the pair recurrence's exchange words (n 64-bit words) before a launch.
+// Zeroes a run's exchange words (n 64-bit words).
 __global__ void __launch_bounds__(256) lstm_exchange_clear_kernel(uint64_t* x, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) x[i] = 0;
@@ -839,37 +886,37 @@ hipError_t launch_lstm_pair(const float* gx, int64_t gx_ld, const int32_t* gx_ro
         attr_set.fetch_or(1ull << dev);
     }
     const int nseq = 2 * nb;
-    const int64_t words = (int64_t)nseq * 512;
-    hipLaunchKernelGGL(lstm_exchange_clear_kernel, dim3((unsigned)ceil_div(words, 256)), dim3(256), 0, s, xbuf, words);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(lstm_pair_kernel, dim3((unsigned)(ceil_div(nseq, 8) * 16)), dim3(kLstmThreads), kLpLds, s, gx,
                        gx_ld, gx_row, start, len, nseq, whh_t, bhh, out, out_ld, xbuf, abort, wait_ticks, silent_half);
     return hipGetLastError();
 }
 
-hipError_t launch_lstm_quad(const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start,
-                            const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
-                            float* out, int64_t out_ld, uint64_t* xbuf, int* abort, hipStream_t s, uint64_t wait_ticks,
-                            int silent_quarter) {
+hipError_t launch_lstm_split(int parts, const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start,
+                             const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
+                             float* out, int64_t out_ld, uint64_t* xbuf, int* abort, hipStream_t s, uint64_t wait_ticks,
+                             int silent_part) {
     if (nb <= 0) return hipSuccess;
-    if (!xbuf || !abort || !sched || wait_ticks == 0) return hipErrorInvalidValue;
-    const int nseq = 2 * nb, nq = lstm_quads(nb);
-    const int64_t words = (int64_t)nseq * 512;
-    hipLaunchKernelGGL(lstm_exchange_clear_kernel, dim3((unsigned)ceil_div(words, 256)), dim3(256), 0, s, xbuf, words);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(lstm_quad_kernel, dim3((unsigned)(ceil_div(nq, 8) * 32)), dim3(kLstmThreads), 0, s, gx, gx_ld,
-                       gx_row, start, len, sched, nq, whh_t, bhh, out, out_ld, xbuf, abort, wait_ticks, silent_quarter);
-    return hipGetLastError();
+    const int nq = lstm_groups(nb);
+    if (!xbuf || !abort || !sched || wait_ticks == 0 || parts * nq > 256) return hipErrorInvalidValue;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)(ceil_div(nq, 8) * 8 * parts)), dim3(kLstmThreads), 0, s, gx, gx_ld, gx_row,
+                           start, len, sched, nq, whh_t, bhh, out, out_ld, xbuf, abort, wait_ticks, silent_part);
+        return hipGetLastError();
+    };
+    switch (parts) {
+        case 4: return go(lstm_split_kernel<4>);
+        case 8: return go(lstm_split_kernel<8>);
+        case 16: return go(lstm_split_kernel<16>);
+    }
+    return hipErrorInvalidValue;
 }
 
 std::vector<int32_t> lstm_schedule(const int64_t* len, int nb) {
-    const int nq = lstm_quads(nb);
+    const int nq = lstm_groups(nb);
     std::vector<int32_t> items(nb);
     for (int i = 0; i < nb; i++) items[i] = i;
     std::stable_sort(items.begin(), items.end(), [&](int a, int b) { return len[a] > len[b]; });
-    typedef std::pair<int64_t, int> Load;  // (total length, quad): the least first, ties by quad
+    typedef std::pair<int64_t, int> Load;  // (total length, group): the least first, ties by group
     std::priority_queue<Load, std::vector<Load>, std::greater<Load>> free_q;
     for (int q = 0; q < nq; q++) free_q.push(Load{0, q});
     std::vector<std::vector<int32_t>> lists(nq);

@@ -1,0 +1,33 @@
+"""The BiLSTM recurrences on 16, 8 and 4 CUs per sequence (chosen by the number of sequences), against the
+two-CU kernel (KOKORO_HIP_LSTM_QUAD=0): each row's sums are in the same order, so durations and audio
+must be equal bit for bit; batch sizes on either side of every boundary (2 nb = 16, 32, 64 sequences)
+and past the last, where groups run lists of sequences."""
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nb", [1, 8, 9, 16, 17, 32, 33])
+def test_split_matches_pair(nb):
+    from kokoro_hip import api, model_spec, workloads
+    ctx = api.Context(0)
+    ctx.upload_model(model_spec.random_model_weights(seed=0))
+    rng = np.random.default_rng(nb)
+    items = workloads.small_ids_items(90 + nb, [int(n) for n in rng.integers(1, 24, nb)])
+    res = {}
+    for sel in ("1", "0", None):
+        if sel is None:
+            os.environ.pop("KOKORO_HIP_LSTM_QUAD", None)
+        else:
+            os.environ["KOKORO_HIP_LSTM_QUAD"] = sel
+        try:
+            res[sel] = ctx.forward_batch(items)
+        finally:
+            os.environ.pop("KOKORO_HIP_LSTM_QUAD", None)
+    for sel in ("1", None):
+        for b, ((a, d), (a2, d2)) in enumerate(zip(res[sel], res["0"])):
+            assert np.array_equal(d, d2) and np.array_equal(a, a2), (sel, b)
+    ctx.close()
