@@ -699,10 +699,9 @@ hipError_t launch_t(const ConvParams& p, int n_cu, hipStream_t s, bool validate_
         return hipErrorInvalidValue;
     if (p.tile_wn != WN) return hipErrorInvalidValue;
     if (validate_only) return hipSuccess;
-    // Launches of few units on the narrow kernel (not the layers of at most 32 rows, nor the
-    // (PRO_LEAKY, EPI_STORE) layers, which it has no variants of; only Snake layers have large halos)
-    if constexpr (MI == 2 && !(PRO == PRO_LEAKY && EPI == EPI_STORE)) {
-        if (conv_units64(p) <= kNarrowUnits && (PRO == PRO_ADAIN_SNAKE || halo <= kSmallHalo)) {
+    static_assert(kNarrowHalo == kSmallHalo, "the narrow kernel's halos");
+    if constexpr (MI == 2 && !(PRO == PRO_LEAKY && EPI == EPI_STORE)) {  // launches of few units
+        if (conv_narrow(p, PRO, EPI, SHAPE_256x128)) {
             ConvGroup g{};
             g.n = 1, g.p[0] = p;
             return launch_conv_narrow(g, PRO, EPI, STATS, IN_H, OUT_H, s);

@@ -1373,6 +1373,18 @@ struct Runner {
                                    xrow_at);
         });
     }
+    // n (<= kFinMaxOuts) tensors of one shape, their partials in regions 0 .. n - 1: one launch.
+    void fin_each(const Tiles& t, int wn, int c, int n, const MAdain* const* as, Coef* const* cs) {
+        check(n >= 1 && n <= kFinMaxOuts, "finalize outputs");
+        FinOuts fo{};
+        fo.n = n;
+        for (int k = 0; k < n; k++) fo.o[k] = FinOut{as[k]->gb_off, as[k]->nw.as<float>(), as[k]->nb.as<float>(), cs[k]};
+        const double bytes = (double)n * ((double)t.count * wn * c * sizeof(StatPart) + (double)p->nb * c * (sizeof(Coef) + 8));
+        launch(PC_FINALIZE, 0, bytes, [&] {
+            return launch_finalize(p->part.as<StatPart>(), c, wn, t.dev(), p->nb, t.max_tiles * wn, gbuf(), gb_ld(), fo, s,
+                                   nullptr, 0, nullptr, p->part_bytes / (int64_t)sizeof(StatPart));
+        });
+    }
     void stats_fin(const float* x, int64_t ld, int c, const Dom& d, const MAdain& a, Coef* coef) {
         fin(stats(x, ld, c, d), 1, c, a, coef);
     }
@@ -1401,10 +1413,15 @@ struct Runner {
         int stride = 1, pad_t = 0;
         bool in_h = false, out_h = false;  // fp16 input / output (the Snake steps' h)
     };
-    const Tiles& conv(const MConv& c, const Op& o) {
+    // The launch parameters of a layer, its tiles, and its algorithmic FLOP and bytes (added to the
+    // run's); the dry run validates them.
+    struct Cost {
+        double f, bytes;
+    };
+    const Tiles& prep(const MConv& c, const Op& o, ConvParams& q, Cost& cost) {
         const int wn = kShapeWN[c.shape], bn = kShapeN[c.shape];
         const Tiles& t = o.convt ? p->tl(*o.din, bn, 1) : p->tl(*o.dout, bn);
-        ConvParams q{};
+        q = ConvParams{};
         q.x = o.x, q.x_ld = o.x_ld, q.l_in = o.din->l, q.cin = c.cin, q.cin_pad = c.cin_pad;
         q.in_max_len = o.din->len.empty() ? 0 : *std::max_element(o.din->len.begin(), o.din->len.end());
         q.in_start = o.din->start_d.as<int64_t>(), q.in_len = o.din->len_d.as<int64_t>();
@@ -1454,10 +1471,65 @@ struct Runner {
             if (launch_conv(q, o.pro, o.epi, c.shape, o.stats, o.in_h, o.out_h, ctx->n_cu, s, true) != hipSuccess)
                 fail(KK_ERR_INVALID, "convolution parameters out of the kernel's range (batch too large?)");
         }
+        cost = Cost{f, bytes};
+        return t;
+    }
+    const Tiles& conv(const MConv& c, const Op& o) {
+        ConvParams q;
+        Cost cost;
+        const Tiles& t = prep(c, o, q, cost);
         label = o.label;
-        launch(o.cls, f, bytes,
+        launch(o.cls, cost.f, cost.bytes,
                [&] { return launch_conv(q, o.pro, o.epi, c.shape, o.stats, o.in_h, o.out_h, ctx->n_cu, s); });
         return t;
+    }
+    // n layers that differ only in sizes, operands and weights (one prologue, epilogue and set of
+    // types; none reads another's output), each with its statistics region: one launch when every
+    // one of them is the narrow kernel's, else one after another.
+    struct GroupOp {
+        const MConv* c;
+        Op o;
+        int region;
+    };
+    bool groupable(const GroupOp* g, int n) {
+        if (ctx->profiling || dry || n < 2 || n > kConvGroup) return false;
+        for (int i = 0; i < n; i++) {
+            const Op& o = g[i].o;
+            const Op& o0 = g[0].o;
+            if (o.pro != o0.pro || o.epi != o0.epi || o.stats != o0.stats || o.in_h != o0.in_h || o.out_h != o0.out_h ||
+                o.convt || o.t_hi >= 0)
+                return false;
+            ConvParams q{};
+            const Tiles& t = p->tl(*o.dout, kShapeN[g[i].c->shape]);
+            q.tiles.count = t.count, q.tile_wn = kShapeWN[g[i].c->shape], q.m_pad = g[i].c->m_pad;
+            q.k = g[i].c->k, q.dil = g[i].c->dil;
+            if (!conv_narrow(q, o.pro, o.epi, g[i].c->shape)) return false;
+        }
+        return true;
+    }
+    void conv_group(const GroupOp* g, int n) {
+        const int reg = region;
+        if (groupable(g, n)) {
+            ConvGroup cg{};
+            Cost sum{0, 0};
+            cg.n = n;
+            for (int i = 0; i < n; i++) {
+                Cost cost;
+                region = g[i].region;
+                prep(*g[i].c, g[i].o, cg.p[i], cost);
+                sum.f += cost.f, sum.bytes += cost.bytes;
+            }
+            const Op& o = g[0].o;
+            label = o.label;
+            launch(o.cls, sum.f, sum.bytes,
+                   [&] { return launch_conv_narrow(cg, o.pro, o.epi, o.stats, o.in_h, o.out_h, s); });
+        } else {
+            for (int i = 0; i < n; i++) {
+                region = g[i].region;
+                conv(*g[i].c, g[i].o);
+            }
+        }
+        region = reg;
     }
 
     Op snake_op(const MSnake& blk, const Dom& d, const void* x, float* y, int epi, const Coef* coef, int i,
@@ -1518,6 +1590,7 @@ struct Runner {
         const MAdain* a1s[3] = {&rbs[0].a1[0], &rbs[1].a1[0], &rbs[2].a1[0]};
         Coef* const c1s[3] = {cf(2), cf(3), cf(4)};
         fin_n(yt, yparts, c, 3, a1s, c1s, y_refl ? y : nullptr, y_refl ? d.start_d.as<int64_t>() : nullptr);
+        if (resblocks_grouped(rbs, y, X, hs, d, post_out, post_slope)) return;
         // The three blocks are independent until the mean: blocks 0 and 1 run on the context's
         // side streams and block 2 on the main stream, each with its own h, statistics region and
         // AdaIN coefficients, and the mean (block 2's last conv) waits for the other two.  One
@@ -1572,6 +1645,50 @@ struct Runner {
             conv(rbs[2].c2[2], mean_op);
         }
         s = main_s, region = 0;
+    }
+
+    // The same steps with the three blocks' convolutions of a step in one launch (the longest kernel
+    // first, so that its blocks start first) and their AdaINs in one, when the layers are the narrow
+    // kernel's: 14 launches per stage instead of 36, and no streams to fork and join (a wait for
+    // another stream's event costs 10-20 us, a launch ~4 us of host time).  A 40-frame item's stage
+    // takes ~120 us instead of ~210.  False, and nothing launched, for other sizes.
+    bool resblocks_grouped(const MSnake* rbs, const uint16_t* y, float* X[3], float* const hs[3], const Dom& d,
+                           void* post_out, float post_slope) {
+        const int c = rbs[0].c, wn = kShapeWN[rbs[0].c1[0].shape];
+        const Tiles& t = p->tl(d, kShapeN[rbs[0].c1[0].shape]);
+        Coef* const ca[3] = {cf(5), cf(7), cf(0)};  // the steps' AdaIN pairs
+        Coef* const cb[3] = {cf(6), cf(8), cf(1)};
+        for (int i = 0; i < 3; i++) {
+            GroupOp g1[3], g2[3];
+            for (int k = 0; k < 3; k++) {
+                const int j = 2 - k;
+                const MSnake& blk = rbs[j];
+                Op o1 = snake_op(blk, d, i == 0 ? (const void*)y : X[j], hs[j], EPI_STORE, i == 0 ? cf(2 + j) : ca[j], i,
+                                 false, true);
+                o1.in_h = true;
+                g1[k] = GroupOp{&blk.c1[i], o1, j};
+                Op o2 = snake_op(blk, d, hs[j], X[j], EPI_ACCUM, cb[j], i, true, i < 2);
+                o2.out_h = true;
+                if (i == 0) o2.epi = EPI_ADD_FROM, o2.r0 = (const float*)y, o2.r0_ld = c;
+                g2[k] = GroupOp{&blk.c2[i], o2, j};
+            }
+            if (i == 0 && !groupable(g1, 3)) return false;
+            conv_group(g1, 3);
+            const MAdain* a2[3] = {&rbs[0].a2[i], &rbs[1].a2[i], &rbs[2].a2[i]};
+            fin_each(t, wn, c, 3, a2, cb);
+            if (i < 2) {
+                conv_group(g2, 3);
+                const MAdain* a1[3] = {&rbs[0].a1[i + 1], &rbs[1].a1[i + 1], &rbs[2].a1[i + 1]};
+                fin_each(t, wn, c, 3, a1, ca);
+            } else {
+                conv_group(g2 + 1, 2);  // blocks 1 and 0; block 2's is the mean, from their sums
+                Op m = g2[0].o;
+                m.epi = EPI_MEAN3_LEAKY_BF16, m.r0 = X[0], m.r1 = X[1], m.r2 = X[2], m.r0_ld = c;
+                m.slope = post_slope, m.y = (float*)post_out;
+                conv(rbs[2].c2[2], m);
+            }
+        }
+        return true;
     }
 
     // AdainResBlk1d (src/gpu_batch.rs:104-135) without upsampling: in [ln][in_ld] -> out[:, 0:dout].
@@ -1689,6 +1806,10 @@ struct Runner {
     // with its own h, statistics region (3) and coefficient pair, so that it can run beside the
     // decoder and the previous stage.
     void noise_branch(int i) {
+        noise_conv(i);
+        noise_resblock(i);
+    }
+    void noise_conv(int i) {
         const Dom& dout = i == 0 ? p->d20 : p->d120;
         const int c = m.ups[i].cout;
         uint16_t* xs = p->xs[i].as<uint16_t>();  // an fp16 stream from the noise conv on
@@ -1705,7 +1826,14 @@ struct Runner {
                                      p->d120.len_d.as<int64_t>(), nc.wp.as<uint16_t>(), nc.b.as<float>(), nc.cout,
                                      nc.k, nc.stride, nc.pad, xs, c, tn.dev(), tile_rows, part(), s);
         });
-        snake_block(m.noise_res[i], xs, p->hn.as<float>(), dout, &tn, cf(9), cf(10), true);
+        region = reg;
+    }
+    void noise_resblock(int i) {
+        const Dom& dout = i == 0 ? p->d20 : p->d120;
+        const int reg = region;
+        region = 3;
+        snake_block(m.noise_res[i], p->xs[i].as<uint16_t>(), p->hn.as<float>(), dout,
+                    &p->tl(dout, i == 0 ? kNoiseTile : kNoiseTile1), cf(9), cf(10), true);
         region = reg;
     }
 
@@ -1808,13 +1936,15 @@ struct Runner {
     void linear(const MLinear& L, const void* x, int64_t x_ld, const Dom& d, void* y, int64_t y_ld,
                 const std::string& name, int pro = PRO_F32, int epi = EPI_STORE) {
         const bool out_h = epi == EPI_GELU_BF16;
+        std::vector<GroupOp> g;
         for (size_t i = 0; i < L.piece.size(); i++) {
             Op o;
             o.pro = pro, o.epi = epi, o.x = x, o.x_ld = x_ld, o.din = o.dout = &d, o.out_h = out_h;
             o.y = (float*)((char*)y + L.col0[i] * (out_h ? 2 : 4));
             o.y_ld = y_ld, o.cls = PC_LINEAR, o.label = name;
-            conv(L.piece[i], o);
+            g.push_back(GroupOp{&L.piece[i], o, region});
         }
+        conv_group(g.data(), (int)g.size());
     }
     // BiLSTM recurrence over the item spans of d (gx rows through gx_row, or the spans' own rows);
     // h into out[row][0:512].  Algorithmic traffic: gx read and h written once per row, W_hh once.
@@ -2086,16 +2216,28 @@ struct Runner {
             KK_HIP(hipStreamWaitEvent(ctx->side[2], p->noise_ev[0], 0));
             s = ctx->side[2];
             source();
-            noise_branch(0);
+            noise_conv(0);
+            s = main_s;
+        }
+        auto noise_rest = [&]() {
+            s = ctx->side[2];
+            noise_resblock(0);
             KK_HIP(hipEventRecord(p->noise_ev[1], s));
             if (until > KK_STAGE_GEN0) {
                 noise_branch(1);
                 KK_HIP(hipEventRecord(p->noise_ev[2], s));
             }
             s = main_s;
-        }
+        };
+        // Short calls: the decoder's launches before the rest of the noise branches', whose 25 launches
+        // kept the main stream idle for ~110 us (of 900 on a 40-frame item).  Calls of more frames
+        // are not bound by the host and fill the GPU with the noise branches while t_en is staged
+        // (13,501 frames: 0.3 to 1% slower the other way round).
+        const bool decoder_first = frames() <= 2048;
+        if (conc && !decoder_first) noise_rest();
         if (p->late_items && !dry) stage_late_ten();
         if (p->kind == PLAN_DECODER || p->kind == PLAN_FULL) decoder();
+        if (conc && decoder_first) noise_rest();
         if (until <= KK_STAGE_DECODER) return;
         if (!conc) source();
         if (until <= KK_STAGE_SOURCE) return;

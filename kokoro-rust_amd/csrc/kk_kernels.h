@@ -114,6 +114,13 @@ hipError_t launch_conv_narrow(ConvGroup& g, int pro, int epi, bool stats, bool i
 // 512, and batches of 1,200 frames 10% at 1,024.
 constexpr int64_t kNarrowUnits = 256;
 inline int64_t conv_units64(const ConvParams& p) { return p.tiles.count * p.tile_wn * (p.m_pad / 64); }
+// Layers it takes (besides: not those of at most 32 rows, nor (PRO_LEAKY, EPI_STORE), which it has no
+// variants of; only Snake layers have large halos).
+constexpr int kNarrowHalo = 16;
+inline bool conv_narrow(const ConvParams& p, int pro, int epi, int shape) {
+    return shape != SHAPE_32x256 && !(pro == PRO_LEAKY && epi == EPI_STORE) && conv_units64(p) <= kNarrowUnits &&
+           (pro == PRO_ADAIN_SNAKE || (p.k - 1) * p.dil <= kNarrowHalo);
+}
 
 // ---------------------------------------------------------------- bandwidth kernels (kk_misc.hip)
 // Statistics partials of x [l][ld] over tiles (one partial per tile and channel).
@@ -137,9 +144,12 @@ struct FinOuts {
     int n;
 };
 // xrow (fp16 [.][xrow_ld]): one more sample per item outside the partials, row xrow_at[b].
+// each_stride != 0: output k is of a tensor of its own, whose partials are each_stride records after
+// output k - 1's (the same steps of several resblocks in one launch).
 hipError_t launch_finalize(const StatPart* part, int c, int wn, TilesDev t, int nb, int64_t max_parts,
                            const float* gb, int64_t gb_ld, const FinOuts& outs, hipStream_t s,
-                           const uint16_t* xrow = nullptr, int64_t xrow_ld = 0, const int64_t* xrow_at = nullptr);
+                           const uint16_t* xrow = nullptr, int64_t xrow_ld = 0, const int64_t* xrow_at = nullptr,
+                           int64_t each_stride = 0);
 // gb[b][j] = W[j] . style[b] + bias[j] for every AdaIN layer at once.
 hipError_t launch_style_fc(const float* w, const float* bias, int rows, const float* style, int nb, float* gb,
                            hipStream_t s);

@@ -74,8 +74,11 @@ template <int SUB, int LOADS>
 __global__ __launch_bounds__(16 * SUB) void finalize_kernel(const StatPart* __restrict__ part, int c, int wn, TilesDev t,
                                                             const float* __restrict__ gb, int64_t gb_ld, FinOuts outs,
                                                             const uint16_t* __restrict__ xrow, int64_t xrow_ld,
-                                                            const int64_t* __restrict__ xrow_at) {
+                                                            const int64_t* __restrict__ xrow_at, int64_t each_stride) {
     constexpr int kFinSub = SUB;
+    // each_stride: block z reduces output z's own partials; else one reduction serves all outputs
+    part += blockIdx.z * each_stride;
+    const int k_lo = each_stride ? blockIdx.z : 0, k_hi = each_stride ? blockIdx.z + 1 : outs.n;
     __shared__ double sa[kFinSub][16], sb[kFinSub][16], sn[kFinSub][16];
     const int cl = threadIdx.x & 15, sub = threadIdx.x >> 4;
     const int b = blockIdx.x;
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(16 * SUB) void finalize_kernel(const StatPart* __re
     if (n <= 0.0) {
 #pragma unroll
         for (int k = 0; k < kFinMaxOuts; k++)
-            if (k < outs.n) outs.o[k].coef[i] = Coef{0.f, 0.f};
+            if (k >= k_lo && k < k_hi) outs.o[k].coef[i] = Coef{0.f, 0.f};
         return;
     }
     const double dm = a1 / n;
@@ -136,7 +139,7 @@ __global__ __launch_bounds__(16 * SUB) void finalize_kernel(const StatPart* __re
     // each AdaIN layer of this tensor: its own style offset, norm weight / bias and coefficients
 #pragma unroll
     for (int k = 0; k < kFinMaxOuts; k++) {
-        if (k >= outs.n) break;
+        if (k < k_lo || k >= k_hi) continue;
         const FinOut& o = outs.o[k];
         const double g1 = 1.0 + (double)gb[b * gb_ld + o.gb_off + ch];
         const double beta = gb[b * gb_ld + o.gb_off + c + ch];
@@ -920,12 +923,12 @@ hipError_t launch_stats_tiles(const float* x, int64_t ld, int c, TilesDev t, Sta
 
 hipError_t launch_finalize(const StatPart* part, int c, int wn, TilesDev t, int nb, int64_t max_parts,
                            const float* gb, int64_t gb_ld, const FinOuts& outs, hipStream_t s, const uint16_t* xrow,
-                           int64_t xrow_ld, const int64_t* xrow_at) {
+                           int64_t xrow_ld, const int64_t* xrow_at, int64_t each_stride) {
     if (outs.n < 1 || outs.n > kFinMaxOuts) return hipErrorInvalidValue;
-    dim3 grid((unsigned)nb, (unsigned)ceil_div(c, 16));
+    dim3 grid((unsigned)nb, (unsigned)ceil_div(c, 16), (unsigned)(each_stride ? outs.n : 1));
     auto go = [&](auto kern, int sub) {
         hipLaunchKernelGGL(kern, grid, dim3(16 * sub), 0, s, part, c, wn, t, gb, gb_ld, outs, xrow, xrow_ld,
-                           xrow_at);
+                           xrow_at, each_stride);
         return hipGetLastError();
     };
     if (max_parts <= 16) return go(finalize_kernel<16, 1>, 16);
