@@ -2046,7 +2046,7 @@ struct Runner {
         // prosody styles: every AdaLayerNorm / AdaIN projection of the predictor
         label = "predictor.style_fc";
         launch(PC_STYLE, 0, (double)u.style_rows * (kStyleDim + 1 + p->nb) * 4, [&] {
-            return launch_style_fc(u.style_wt.as<float>(), u.style_b.as<float>(), u.style_rows,
+            return launch_style_fc(u.style_wt.as<float>(), u.style_b.as<float>(), 0, u.style_rows, u.style_rows,
                                    p->style_pro.as<float>(), p->nb, p->gbp.as<float>(), s);
         });
         // ALBERT (albert_b, src/gpu_batch.rs:423-455)
@@ -2198,9 +2198,17 @@ struct Runner {
             prosody();
             if (until <= KK_STAGE_PROSODY) return;
         }
-        launch(PC_STYLE, 0, (double)m.style_rows * (kStyleDim + 1 + p->nb) * 4, [&] {
-            return launch_style_fc(m.style_wt.as<float>(), m.style_b.as<float>(), m.style_rows, p->style.as<float>(),
-                                   p->nb, p->gb.as<float>(), s);
+        // a Snake block's plan: only the rows of its own AdaINs (a few hundred of the table's 37,504)
+        int row0 = 0, row1 = m.style_rows;
+        if (p->kind == PLAN_SNAKE) {
+            row0 = m.style_rows, row1 = 0;
+            for (int i = 0; i < 3; i++)
+                for (const MAdain* a : {&p->sblk->a1[i], &p->sblk->a2[i]})
+                    row0 = std::min(row0, a->gb_off), row1 = std::max(row1, a->gb_off + 2 * a->c);
+        }
+        launch(PC_STYLE, 0, (double)(row1 - row0) * (kStyleDim + 1 + p->nb) * 4, [&] {
+            return launch_style_fc(m.style_wt.as<float>(), m.style_b.as<float>(), row0, row1 - row0, m.style_rows,
+                                   p->style.as<float>(), p->nb, p->gb.as<float>(), s);
         });
         if (p->kind == PLAN_SNAKE) {
             snake_block(*p->sblk, p->B[0].as<float>(), p->B[1].as<float>(), p->ds);

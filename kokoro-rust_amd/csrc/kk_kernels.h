@@ -151,8 +151,8 @@ hipError_t launch_finalize(const StatPart* part, int c, int wn, TilesDev t, int 
                            const uint16_t* xrow = nullptr, int64_t xrow_ld = 0, const int64_t* xrow_at = nullptr,
                            int64_t each_stride = 0);
 // gb[b][j] = W[j] . style[b] + bias[j] for every AdaIN layer at once.
-hipError_t launch_style_fc(const float* w, const float* bias, int rows, const float* style, int nb, float* gb,
-                           hipStream_t s);
+hipError_t launch_style_fc(const float* w, const float* bias, int row0, int rows, int ld, const float* style, int nb,
+                           float* gb, hipStream_t s);
 // asr[t][c] = t_en[src_row[t]][c] (0 in gaps): t_en token rows [t_rows][512] -> frame rows [l][ld],
 // channels [0, 512).
 hipError_t launch_expand(const float* t_en, int64_t t_rows, const int32_t* src_row, int64_t l, float* asr,

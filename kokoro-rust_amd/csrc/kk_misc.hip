@@ -150,43 +150,54 @@ __global__ __launch_bounds__(16 * SUB) void finalize_kernel(const StatPart* __re
 
 // ------------------------------------------------------------------ style projections
 // GLinear of every AdaIN (src/gpu_batch.rs:84): gb[b][j] = bias[j] + sum_k W[j][k] style[b][k], summed
-// in f64.  W is stored transposed [128][rows] so consecutive threads read consecutive rows.  A block
+// in f64.  W is stored transposed [128][ld] so consecutive threads read consecutive rows.  A block
 // covers 64 rows; its four waves take one quarter of k each (the loads of a quarter issued
-// together), and the quarters' sums meet in LDS, 16 items per pass.
+// together), and the quarters' sums meet in LDS, E items per pass.  Bound by the table's read (the
+// decoder's and generator's 37,504 rows: 19 MB) and, from a few items on, by the f64 sums: E is the
+// smallest of 1, 4 and 16 that holds the batch, as sums of items that are not there cost as much as
+// real ones.  Of few rows (kStyleFewRows; one Snake block's AdaINs) the passes run in blocks of 4
+// items each beside each other, reading the rows again from the L2.  Measured
+// (one pass of 16 sums over the whole table for every call before): one item, all rows, 14 -> 9 us;
+// one block's rows, 16 items as one pass of 16, 10 us; the one-block calls on device memory, whole
+// call: 1 item 206 -> 162 us (with the convolutions' gains), 16 ragged items 406 -> 391 us.
+constexpr int kStyleFewRows = 4096;
+template <int E>
 __global__ __launch_bounds__(256) void style_fc_kernel(const float* __restrict__ wt, const float* __restrict__ bias,
-                                                       int rows, const float* __restrict__ style, int nb,
-                                                       float* __restrict__ gb) {
-    __shared__ float st[16][kStyleDim];
-    __shared__ double part[3][16][64];
+                                                       int row0, int rows, int ld, const float* __restrict__ style,
+                                                       int nb, float* __restrict__ gb) {
+    __shared__ float st[E][kStyleDim];
+    __shared__ double part[3][E][64];
     const int r = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int j = blockIdx.x * 64 + r;
-    const int jc = j < rows ? j : rows - 1;
+    const int jl = blockIdx.x * 64 + r;
+    const int j = row0 + (jl < rows ? jl : rows - 1);
     float w[32];
 #pragma unroll
-    for (int i = 0; i < 32; i++) w[i] = wt[(int64_t)(32 * q + i) * rows + jc];
-    for (int b0 = 0; b0 < nb; b0 += 16) {
-        const int cnt = min(16, nb - b0);
+    for (int i = 0; i < 32; i++) w[i] = wt[(int64_t)(32 * q + i) * ld + j];
+    for (int b0 = E * blockIdx.y; b0 < nb; b0 += E * gridDim.y) {
+        const int cnt = min(E, nb - b0);
         __syncthreads();
-        for (int i = threadIdx.x; i < 16 * kStyleDim; i += 256)
+        for (int i = threadIdx.x; i < E * kStyleDim; i += 256)
             st[i / kStyleDim][i % kStyleDim] = i / kStyleDim < cnt ? style[(int64_t)b0 * kStyleDim + i] : 0.f;
         __syncthreads();
-        double acc[16];
+        double acc[E];
 #pragma unroll
-        for (int e = 0; e < 16; e++) acc[e] = 0.0;
+        for (int e = 0; e < E; e++) acc[e] = 0.0;
 #pragma unroll
         for (int i = 0; i < 32; i++) {
             const double wv = w[i];
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[e] += wv * (double)st[e][32 * q + i];
+            for (int e = 0; e < E; e++) acc[e] += wv * (double)st[e][32 * q + i];
         }
         if (q > 0)
 #pragma unroll
-            for (int e = 0; e < 16; e++) part[q - 1][e][r] = acc[e];
+            for (int e = 0; e < E; e++) part[q - 1][e][r] = acc[e];
         __syncthreads();
-        if (q == 0 && j < rows)
-            for (int e = 0; e < cnt; e++)
-                gb[(int64_t)(b0 + e) * rows + j] =
-                    (float)(((acc[e] + part[0][e][r]) + (part[1][e][r] + part[2][e][r])) + (double)bias[j]);
+        if (q == 0 && jl < rows)
+#pragma unroll
+            for (int e = 0; e < E; e++)
+                if (e < cnt)
+                    gb[(int64_t)(b0 + e) * ld + j] =
+                        (float)(((acc[e] + part[0][e][r]) + (part[1][e][r] + part[2][e][r])) + (double)bias[j]);
     }
 }
 
@@ -938,10 +949,15 @@ hipError_t launch_finalize(const StatPart* part, int c, int wn, TilesDev t, int 
     return go(finalize_kernel<64, 8>, 64);
 }
 
-hipError_t launch_style_fc(const float* w, const float* bias, int rows, const float* style, int nb, float* gb,
-                           hipStream_t s) {
+hipError_t launch_style_fc(const float* w, const float* bias, int row0, int rows, int ld, const float* style, int nb,
+                           float* gb, hipStream_t s) {
     if (rows <= 0 || nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL(style_fc_kernel, dim3(blocks_for(rows, 64)), dim3(256), 0, s, w, bias, rows, style, nb, gb);
+    if (row0 < 0 || row0 > ld - rows) return hipErrorInvalidValue;
+    const bool few = rows <= kStyleFewRows;
+    auto kern = nb == 1 ? style_fc_kernel<1> : nb <= 4 || few ? style_fc_kernel<4> : style_fc_kernel<16>;
+    const unsigned passes = few && nb > 4 ? (unsigned)std::min<int64_t>(ceil_div(nb, 4), 4096) : 1;
+    hipLaunchKernelGGL(kern, dim3(blocks_for(rows, 64), passes), dim3(256), 0, s, w, bias, row0, rows, ld, style, nb,
+                       gb);
     return hipGetLastError();
 }
 
