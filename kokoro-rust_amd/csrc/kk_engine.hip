@@ -1391,7 +1391,17 @@ struct Runner {
         });
     }
     void stats_fin(const float* x, int64_t ld, int c, const Dom& d, const MAdain& a, Coef* coef) {
-        fin(stats(x, ld, c, d), 1, c, a, coef);
+        const Tiles& t = p->tl(d, kStatTile);
+        if (t.max_tiles > kStatFinTiles || ctx->profiling || dry) {
+            fin(stats(x, ld, c, d), 1, c, a, coef);
+            return;
+        }
+        // items of few tiles: one launch
+        FinOuts fo{};
+        fo.n = 1, fo.o[0] = FinOut{a.gb_off, a.nw.as<float>(), a.nb.as<float>(), coef};
+        launch(PC_STATS, 0, (double)d.valid() * c * 4 + (double)p->nb * c * (sizeof(Coef) + 8), [&] {
+            return launch_stats_fin(x, ld, c, t.dev(), p->nb, t.max_tiles, gbuf(), gb_ld(), fo, s);
+        });
     }
 
     // One MFMA conv launch.

@@ -150,6 +150,10 @@ hipError_t launch_finalize(const StatPart* part, int c, int wn, TilesDev t, int 
                            const float* gb, int64_t gb_ld, const FinOuts& outs, hipStream_t s,
                            const uint16_t* xrow = nullptr, int64_t xrow_ld = 0, const int64_t* xrow_at = nullptr,
                            int64_t each_stride = 0);
+// launch_stats_tiles and launch_finalize in one launch, items of at most kStatFinTiles tiles.
+constexpr int kStatFinTiles = 4;
+hipError_t launch_stats_fin(const float* x, int64_t ld, int c, TilesDev t, int nb, int64_t max_tiles, const float* gb,
+                            int64_t gb_ld, const FinOuts& outs, hipStream_t s);
 // gb[b][j] = W[j] . style[b] + bias[j] for every AdaIN layer at once.
 hipError_t launch_style_fc(const float* w, const float* bias, int row0, int rows, int ld, const float* style, int nb,
                            float* gb, hipStream_t s);

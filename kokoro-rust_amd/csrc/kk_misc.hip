@@ -30,6 +30,19 @@ __device__ __forceinline__ uint2 pack_f16x4(float4 v) {
 // Statistics partials of x over item-aligned tiles: per (tile, channel) the sums of (v - shift) and
 // (v - shift)^2 with shift = the tile's first value (the centring of chan_stats_seg,
 // kernels/kokoro.cu:779-810, applied per tile).  One wave per 64 channels and row phase.
+// Row phase g of a tile: rows t0 + g, t0 + g + 4, ... of channel ch, U loads in flight.
+template <int U>
+__device__ __forceinline__ void tile_sums(const float* __restrict__ x, int64_t ld, int ch, int64_t t0, int n, int g,
+                                          float& shift, float& s1, float& s2) {
+    shift = x[t0 * ld + ch], s1 = 0.f, s2 = 0.f;
+#pragma unroll U
+    for (int r = g; r < n; r += 4) {
+        const float d = x[(t0 + r) * ld + ch] - shift;
+        s1 += d;
+        s2 = __builtin_fmaf(d, d, s2);
+    }
+}
+
 __global__ __launch_bounds__(256) void stats_tiles_kernel(const float* __restrict__ x, int64_t ld, int c, TilesDev t,
                                                           StatPart* __restrict__ part) {
     __shared__ float sa[4][64], sb[4][64];
@@ -39,15 +52,7 @@ __global__ __launch_bounds__(256) void stats_tiles_kernel(const float* __restric
     const int64_t t0 = t.t0[tile];
     const int n = t.n[tile];
     float shift = 0.f, s1 = 0.f, s2 = 0.f;
-    if (ch < c) {
-        shift = x[t0 * ld + ch];
-#pragma unroll 8
-        for (int r = g; r < n; r += 4) {
-            const float d = x[(t0 + r) * ld + ch] - shift;
-            s1 += d;
-            s2 = __builtin_fmaf(d, d, s2);
-        }
-    }
+    if (ch < c) tile_sums<8>(x, ld, ch, t0, n, g, shift, s1, s2);
     sa[g][lane] = s1;
     sb[g][lane] = s2;
     __syncthreads();
@@ -55,6 +60,44 @@ __global__ __launch_bounds__(256) void stats_tiles_kernel(const float* __restric
         s1 = ((sa[0][lane] + sa[1][lane]) + sa[2][lane]) + sa[3][lane];
         s2 = ((sb[0][lane] + sb[1][lane]) + sb[2][lane]) + sb[3][lane];
         part[tile * c + ch] = StatPart{s1, s2, shift, (float)n};
+    }
+}
+
+// Adds partial q to an item's sums of (v - ref) and (v - ref)^2.
+__device__ __forceinline__ void fin_add(const StatPart& q, double ref, double& a1, double& a2, double& n) {
+    if (q.n > 0.f) {
+        const double dn = (double)q.n, d = (double)q.shift - ref, s1 = (double)q.s1;
+        a1 += s1 + dn * d;
+        a2 += (double)q.s2 + 2.0 * d * s1 + dn * d * d;
+        n += dn;
+    }
+}
+
+// Outputs [k_lo, k_hi)'s coefficients of (item b, channel ch) from its sums.
+__device__ __forceinline__ void fin_coefs(double a1, double a2, double n, double ref, int b, int ch, int c,
+                                          const float* __restrict__ gb, int64_t gb_ld, const FinOuts& outs, int k_lo,
+                                          int k_hi) {
+    const int64_t i = (int64_t)b * c + ch;
+    if (n <= 0.0) {
+#pragma unroll
+        for (int k = 0; k < kFinMaxOuts; k++)
+            if (k >= k_lo && k < k_hi) outs.o[k].coef[i] = Coef{0.f, 0.f};
+        return;
+    }
+    const double dm = a1 / n;
+    double var = a2 / n - dm * dm;
+    if (var < 0.0) var = 0.0;
+    const float meanf = (float)(ref + dm);
+    const float rstd = 1.0f / sqrtf((float)var + 1e-5f);
+    // each AdaIN layer of this tensor: its own style offset, norm weight / bias and coefficients
+#pragma unroll
+    for (int k = 0; k < kFinMaxOuts; k++) {
+        if (k < k_lo || k >= k_hi) continue;
+        const FinOut& o = outs.o[k];
+        const double g1 = 1.0 + (double)gb[b * gb_ld + o.gb_off + ch];
+        const double beta = gb[b * gb_ld + o.gb_off + c + ch];
+        const double a = (double)rstd * (double)o.nw[ch];
+        o.coef[i] = Coef{(float)(a * g1), (float)(((double)o.nb[ch] - (double)meanf * a) * g1 + beta)};
     }
 }
 
@@ -85,15 +128,6 @@ __global__ __launch_bounds__(16 * SUB) void finalize_kernel(const StatPart* __re
     const int ch = blockIdx.y * 16 + cl;
     const int64_t lo = (int64_t)t.lo[b] * wn, hi = (int64_t)t.hi[b] * wn;
     double a1 = 0.0, a2 = 0.0, n = 0.0, ref = 0.0;
-    auto add = [&](const StatPart& q) {
-        if (q.n > 0.f) {
-            const double dn = (double)q.n, d = (double)q.shift - ref, s1 = (double)q.s1;
-            // sums of (v - ref) and (v - ref)^2 over the partial's columns
-            a1 += s1 + dn * d;
-            a2 += (double)q.s2 + 2.0 * d * s1 + dn * d * d;
-            n += dn;
-        }
-    };
     if (ch < c && lo < hi) {
         ref = (double)part[lo * c + ch].shift;
         // partials lo + sub, lo + sub + SUB, ... in increasing order; past hi a record with n = 0
@@ -105,7 +139,7 @@ __global__ __launch_bounds__(16 * SUB) void finalize_kernel(const StatPart* __re
                 q[j] = pi < hi ? part[pi * c + ch] : StatPart{0.f, 0.f, 0.f, 0.f};
             }
 #pragma unroll
-            for (int j = 0; j < LOADS; j++) add(q[j]);
+            for (int j = 0; j < LOADS; j++) fin_add(q[j], ref, a1, a2, n);
         }
     }
     sa[sub][cl] = a1, sb[sub][cl] = a2, sn[sub][cl] = n;
@@ -124,28 +158,47 @@ __global__ __launch_bounds__(16 * SUB) void finalize_kernel(const StatPart* __re
         const double d = (double)(float)__builtin_bit_cast(_Float16, xrow[xrow_at[b] * xrow_ld + ch]) - ref;
         a1 += d, a2 += d * d, n += 1.0;
     }
-    const int64_t i = (int64_t)b * c + ch;
-    if (n <= 0.0) {
-#pragma unroll
-        for (int k = 0; k < kFinMaxOuts; k++)
-            if (k >= k_lo && k < k_hi) outs.o[k].coef[i] = Coef{0.f, 0.f};
-        return;
+    fin_coefs(a1, a2, n, ref, b, ch, c, gb, gb_ld, outs, k_lo, k_hi);
+}
+
+// stats_tiles_kernel and finalize_kernel in one launch, for one output and items of at most T tiles: a
+// block is one item's 64 channels, four waves per tile (the tile's row phases), and the wave of the
+// first tile and phase combines the tiles in finalize's order -- the same sums, bit for bit.  Bound by
+// latency: a launch of few blocks takes ~4 us whatever it does, and so does the gap before the next.
+// Whole calls, two launches before: a 300-row block 162 -> 158 us, five decoder items of 60 to 500
+// frames 2.31 -> 2.20 ms, 32 of 100 to 800 the same.  Four tiles: one block's 16 waves; more tiles fill
+// the GPU better as blocks of their own.
+template <int T>
+__global__ __launch_bounds__(256 * T) void stats_fin_kernel(const float* __restrict__ x, int64_t ld, int c, TilesDev t,
+                                                            const float* __restrict__ gb, int64_t gb_ld, FinOuts outs) {
+    __shared__ float sa[T][4][64], sb[T][4][64], ss[T][64];
+    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6 & 3, w = threadIdx.x >> 8;
+    const int b = blockIdx.x, ch = blockIdx.y * 64 + lane;
+    const int lo = t.lo[b], nt = t.hi[b] - lo;
+    if (ch < c && w < nt) {
+        float shift, s1, s2;
+        tile_sums<16>(x, ld, ch, t.t0[lo + w], t.n[lo + w], g, shift, s1, s2);
+        sa[w][g][lane] = s1, sb[w][g][lane] = s2;
+        if (g == 0) ss[w][lane] = shift;
     }
-    const double dm = a1 / n;
-    double var = a2 / n - dm * dm;
-    if (var < 0.0) var = 0.0;
-    const float meanf = (float)(ref + dm);
-    const float rstd = 1.0f / sqrtf((float)var + 1e-5f);
-    // each AdaIN layer of this tensor: its own style offset, norm weight / bias and coefficients
+    __syncthreads();
+    if (threadIdx.x >= 64 || ch >= c) return;
+    double a1[T], a2[T], n[T];
+    const double ref = nt > 0 ? (double)ss[0][lane] : 0.0;
 #pragma unroll
-    for (int k = 0; k < kFinMaxOuts; k++) {
-        if (k < k_lo || k >= k_hi) continue;
-        const FinOut& o = outs.o[k];
-        const double g1 = 1.0 + (double)gb[b * gb_ld + o.gb_off + ch];
-        const double beta = gb[b * gb_ld + o.gb_off + c + ch];
-        const double a = (double)rstd * (double)o.nw[ch];
-        o.coef[i] = Coef{(float)(a * g1), (float)(((double)o.nb[ch] - (double)meanf * a) * g1 + beta)};
+    for (int k = 0; k < T; k++) {
+        a1[k] = 0.0, a2[k] = 0.0, n[k] = 0.0;
+        if (k < nt)
+            fin_add(StatPart{((sa[k][0][lane] + sa[k][1][lane]) + sa[k][2][lane]) + sa[k][3][lane],
+                             ((sb[k][0][lane] + sb[k][1][lane]) + sb[k][2][lane]) + sb[k][3][lane], ss[k][lane],
+                             (float)t.n[lo + k]},
+                    ref, a1[k], a2[k], n[k]);
     }
+#pragma unroll
+    for (int k = T / 2; k > 0; k >>= 1)
+#pragma unroll
+        for (int i = 0; i < k; i++) a1[i] += a1[i + k], a2[i] += a2[i + k], n[i] += n[i + k];
+    fin_coefs(a1[0], a2[0], n[0], ref, b, ch, c, gb, gb_ld, outs, 0, outs.n);
 }
 
 // ------------------------------------------------------------------ style projections
@@ -929,6 +982,19 @@ hipError_t launch_stats_tiles(const float* x, int64_t ld, int c, TilesDev t, Sta
     if (t.count == 0) return hipSuccess;
     dim3 grid((unsigned)t.count, (unsigned)ceil_div(c, 64));
     hipLaunchKernelGGL(stats_tiles_kernel, grid, dim3(256), 0, s, x, ld, c, t, part);
+    return hipGetLastError();
+}
+
+hipError_t launch_stats_fin(const float* x, int64_t ld, int c, TilesDev t, int nb, int64_t max_tiles, const float* gb,
+                            int64_t gb_ld, const FinOuts& outs, hipStream_t s) {
+    if (outs.n < 1 || outs.n > kFinMaxOuts || max_tiles > kStatFinTiles) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)nb, (unsigned)ceil_div(c, 64));
+    if (max_tiles <= 1)
+        hipLaunchKernelGGL(stats_fin_kernel<1>, grid, dim3(256), 0, s, x, ld, c, t, gb, gb_ld, outs);
+    else if (max_tiles <= 2)
+        hipLaunchKernelGGL(stats_fin_kernel<2>, grid, dim3(512), 0, s, x, ld, c, t, gb, gb_ld, outs);
+    else
+        hipLaunchKernelGGL(stats_fin_kernel<4>, grid, dim3(1024), 0, s, x, ld, c, t, gb, gb_ld, outs);
     return hipGetLastError();
 }
 
