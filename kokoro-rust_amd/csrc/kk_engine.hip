@@ -1963,10 +1963,8 @@ struct Runner {
     }
     // BiLSTM recurrence over the item spans of d (gx rows through gx_row, or the spans' own rows);
     // h into out[row][0:512].  Algorithmic traffic: gx read and h written once per row, W_hh once.
-    // Each sequence runs on 16, 8 or 4 CUs (launch_lstm_split; lstm_parts: as many as 256 CUs hold for
-    // every sequence at once) when all the sequences run at once, and on groups of 4 with scheduled
-    // lists when the longest span has at least kLstmQuadMinSteps steps; else on two (launch_lstm_pair;
-    // bit-identical).  `region`: the launch's exchange words, its own within a run (tokens() clears
+    // Each sequence runs on 16, 8 or 4 CUs (launch_lstm_split) or on two (launch_lstm_pair), as
+    // lstm_parts says; bit-identical.  `region`: the launch's exchange words, its own within a run (tokens() clears
     // them all).  KOKORO_HIP_LSTM_SINGLE=1 selects the one-CU kernel (W_hh partly streamed from L2
     // each step), as does a plan whose pairs or groups gave up before (lstm_single).  Test hook, read
     // at each launch: KOKORO_HIP_TEST_LSTM_SILENT=1 keeps the second half of every pair (the second
@@ -1975,13 +1973,13 @@ struct Runner {
     void recur(const MLstm& l, const float* gx, const int32_t* gx_row, const Dom& d, float* out, int64_t out_ld,
                const std::string& name, int region) {
         static const bool single = env_i64("KOKORO_HIP_LSTM_SINGLE", 0) != 0;
-        // KOKORO_HIP_LSTM_QUAD, read at each launch: 1 groups, 0 pairs for every span
+        // KOKORO_HIP_LSTM_QUAD, read at each launch: 1 groups (where they fit the device), 0 pairs for
+        // every span
         check((int)d.len.size() == p->nb, "internal: recurrence domain");
         const int32_t* sched = p->lstm_sched_of(d);
         int64_t longest = 0;
         for (int64_t v : d.len) longest = std::max(longest, v);
-        const int64_t qsel = env_i64("KOKORO_HIP_LSTM_QUAD", -1);
-        const bool split = qsel < 0 ? 2 * p->nb <= kLstmGroups || longest >= kLstmQuadMinSteps : qsel != 0;
+        const int parts = lstm_parts(p->nb, longest, ctx->n_cu, env_i64("KOKORO_HIP_LSTM_QUAD", -1));
         const bool silent = env_i64("KOKORO_HIP_TEST_LSTM_SILENT", 0) != 0;
         const double v = (double)d.valid();
         label = name;
@@ -1991,8 +1989,8 @@ struct Runner {
                                    l.whh_t.as<float>(), l.bhh.as<float>(), out, out_ld, s);
             uint64_t* x = p->u_lstmx.as<uint64_t>();
             uint64_t* words = x + kk_plan::kLstmXHead + (int64_t)region * 2 * p->nb * 512;
-            if (split)
-                return launch_lstm_split(lstm_parts(p->nb), gx, 2048, gx_row, d.start_d.as<int64_t>(),
+            if (parts > 2)
+                return launch_lstm_split(parts, ctx->n_cu, gx, 2048, gx_row, d.start_d.as<int64_t>(),
                                          d.len_d.as<int64_t>(), p->nb, sched, l.whh_t.as<float>(), l.bhh.as<float>(),
                                          out, out_ld, words, (int*)x, s, silent ? 1000 : kLstmPairWaitTicks,
                                          silent ? 1 : -1);

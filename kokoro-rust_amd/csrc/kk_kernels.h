@@ -1,6 +1,7 @@
 // kk_kernels.h -- launch interface of the gfx950 kernels (host side of kk_conv.hip / kk_misc.hip).
 #pragma once
 #include "kk_common.h"
+#include "kk_lstm.h"
 
 #include <vector>
 
@@ -273,22 +274,18 @@ hipError_t launch_lstm_pair(const float* gx, int64_t gx_ld, const int32_t* gx_ro
                             const int64_t* len, int nb, const float* whh_t, const float* bhh, float* out, int64_t out_ld,
                             uint64_t* xbuf, int* abort, hipStream_t s, uint64_t wait_ticks = kLstmPairWaitTicks,
                             int silent_half = -1);
-// `parts` = 4, 8 or 16 CUs per (item, direction), each with its share of h and of the W_hh rows in
-// registers; the same arguments, bit-identical outputs.  lstm_groups(nb) groups of `parts` blocks (at
-// most 256 blocks, one per CU) run the 2 nb sequences as lists, sched = lstm_schedule(len, nb): [nq + 1] offsets, then
-// the sequence ids (2 item + direction) of each group's list.  silent_part >= 0 (a test hook) keeps
-// that part of every group from publishing.
-constexpr int kLstmGroups = 64;              // of 4 blocks: 256 CUs
-constexpr int64_t kLstmQuadMinSteps = 1024;  // past 64 sequences: groups when a span has this many steps, else pairs
-inline int lstm_groups(int nb) { return 2 * nb < kLstmGroups ? 2 * nb : kLstmGroups; }
-// The most CUs per sequence that 256 hold at once: the fewer sequences, the shorter a step.
-inline int lstm_parts(int nb) { return lstm_groups(nb) <= 16 ? 16 : lstm_groups(nb) <= 32 ? 8 : 4; }
 // Longest processing time first: the sequences by decreasing length (items by length, ties by
 // index, both directions in turn), each to the group with the least total length so far (ties: the
 // lowest group).
 std::vector<int32_t> lstm_schedule(const int64_t* len, int nb);
-hipError_t launch_lstm_split(int parts, const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start,
-                             const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
+// `parts` = 4, 8 or 16 CUs per (item, direction), each with its share of h and of the W_hh rows in
+// registers; the same arguments, bit-identical outputs.  `parts` is lstm_parts' choice for a device of
+// n_cu CUs (refused unless lstm_fits).  lstm_groups(nb) groups of `parts` blocks run the 2 nb sequences
+// as lists, sched = lstm_schedule(len, nb): [nq + 1] offsets, then the sequence ids
+// (2 item + direction) of each group's list.  silent_part >= 0 (a test hook) keeps that part of every
+// group from publishing.
+hipError_t launch_lstm_split(int parts, int n_cu, const float* gx, int64_t gx_ld, const int32_t* gx_row,
+                             const int64_t* start, const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
                              float* out, int64_t out_ld, uint64_t* xbuf, int* abort, hipStream_t s,
                              uint64_t wait_ticks = kLstmPairWaitTicks, int silent_part = -1);
 // Zeroes n 64-bit words.

@@ -603,14 +603,13 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_pair_kernel(const float* gx
 //   word's way through the XCD's L2 (0.27 us measured between two blocks of one XCD, 0.37 across),
 //   two transcendental evaluations and three barriers.
 // The parts of a sequence are blocks 8 apart (the same XCD under round-robin dispatch) and 8 P
-// consecutive blocks hold 8 complete sequences; a launch has at most 256 blocks (one per CU), and
-// each group of P blocks runs a list of sequences one after another, from a schedule the host
-// computes at plan creation: longest first, each sequence to the group with the least work so far --
-// the longest start at once, and the short ones follow on the groups that finish first, with no
-// second wave of blocks waiting for CUs.  A group reloads its W_hh rows only when the direction
-// changes; every sequence starts from h = c = 0 and has its own exchange words.  A block whose
-// partners are not resident yet waits for CUs that finishing groups release (nothing a group waits
-// for depends on a later one).  Every wait is bounded as in the pair kernel.
+// consecutive blocks hold 8 complete sequences.  Each group of P blocks runs a list of sequences one
+// after another, from a schedule the host computes at plan creation: longest first, each sequence to
+// the group with the least work so far -- the longest start at once, and the short ones follow on the
+// groups that finish first.  A group reloads its W_hh rows only when the direction changes; every
+// sequence starts from h = c = 0 and has its own exchange words.  A block whose partners are not
+// resident yet waits for slots that finishing groups release; kk_lstm.h says which P leave a slot for
+// them whatever runs beside this launch.  Every wait is bounded as in the pair kernel.
 //   sched: [nq + 1] list offsets, then the sequence ids (2 item + direction) of the groups' lists.
 // acc += w[k + i][e] h[i] for i = 0 .. 15 in sequence, h[i] in lane i of each row of 16 lanes of h: one
 // v_fmac_f32 with a DPP operand each (the compiler makes a move and a multiply-add of it).  The s_nop
@@ -626,8 +625,8 @@ __device__ __forceinline__ void fma16(float& acc, float h, const float (&w)[64][
           "v"(w[k + 12][e]), "v"(w[k + 13][e]), "v"(w[k + 14][e]), "v"(w[k + 15][e]));
 #undef KK_FM
 }
-template <int P>
-__global__ void __launch_bounds__(kLstmThreads) lstm_split_kernel(const float* gx, int64_t gx_ld, const int32_t* gx_row,
+template <int P>  // (two blocks per CU at P = 8 and 16: 4 waves per SIMD; lstm_blocks_per_cu counts on it)
+__global__ void __launch_bounds__(kLstmThreads, 2 * lstm_blocks_per_cu(P)) lstm_split_kernel(const float* gx, int64_t gx_ld, const int32_t* gx_row,
                                                                   const int64_t* start, const int64_t* len,
                                                                   const int32_t* sched, int nq, const float* whh_t,
                                                                   const float* bhh, float* out, int64_t out_ld,
@@ -891,13 +890,13 @@ hipError_t launch_lstm_pair(const float* gx, int64_t gx_ld, const int32_t* gx_ro
     return hipGetLastError();
 }
 
-hipError_t launch_lstm_split(int parts, const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start,
-                             const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
+hipError_t launch_lstm_split(int parts, int n_cu, const float* gx, int64_t gx_ld, const int32_t* gx_row,
+                             const int64_t* start, const int64_t* len, int nb, const int32_t* sched, const float* whh_t, const float* bhh,
                              float* out, int64_t out_ld, uint64_t* xbuf, int* abort, hipStream_t s, uint64_t wait_ticks,
                              int silent_part) {
     if (nb <= 0) return hipSuccess;
     const int nq = lstm_groups(nb);
-    if (!xbuf || !abort || !sched || wait_ticks == 0 || parts * nq > 256) return hipErrorInvalidValue;
+    if (!xbuf || !abort || !sched || wait_ticks == 0 || !lstm_fits(parts, n_cu)) return hipErrorInvalidValue;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)(ceil_div(nq, 8) * 8 * parts)), dim3(kLstmThreads), 0, s, gx, gx_ld, gx_row,
                            start, len, sched, nq, whh_t, bhh, out, out_ld, xbuf, abort, wait_ticks, silent_part);
