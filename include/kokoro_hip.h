@@ -183,9 +183,10 @@ typedef struct {
  * off its CU, e.g. by another process) ends its launch, and the call runs the forward again with
  * the one-CU kernel, which waits on no other block -- contention costs time, not an error (an
  * ids-level plan stays on the one-CU kernel for its later runs; every result path, kk_plan_sync
- * and taps included, runs that check first).  KOKORO_HIP_LSTM_SINGLE=1 (read once per process)
- * selects the one-CU kernel from the start; test hook KOKORO_HIP_TEST_LSTM_SILENT=1 (read at each
- * launch) makes every recurrence give up after a 10 us wait.  ALBERT's attention runs on the f32 matrix cores;
+ * and taps included, runs that check first; the context's later batches run on pairs, which wait for
+ * the fewest blocks).  KOKORO_HIP_LSTM_SINGLE=1 (read once per process) selects the one-CU kernel from
+ * the start; test hook KOKORO_HIP_TEST_LSTM_SILENT=1 (read at each launch) makes every recurrence give
+ * up after a 10 us wait, 2 those on more than two CUs.  ALBERT's attention runs on the f32 matrix cores;
  * KOKORO_HIP_ATTENTION_VALU=1 (read once per process) selects the f32 VALU kernel instead. */
 int kk_forward_batch(kk_ctx* ctx, const kk_item* items, int n, kk_result* out, char* err, size_t errlen);
 void kk_result_free(kk_result* out, int n);

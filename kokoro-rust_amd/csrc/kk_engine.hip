@@ -262,6 +262,8 @@ struct kk_ctx {
     // kk_forward_decoder_batch's plan, kept between calls: its device buffers are reused whenever
     // the next batch fits (released on any failure, so that a split batch can use the memory)
     kk_plan* oneshot = nullptr;
+    // a recurrence of this context gave up: the later batches' by pairs, which wait for fewer blocks
+    bool lstm_pairs = false;
     // device address of this device's copy of the no-allocation entry point's scratch array
     unsigned char* scratch = nullptr;
     // kk_encode_pcm16's device buffer (at most kPcmKeepBytes) and pinned result word, kept between
@@ -1968,19 +1970,21 @@ struct Runner {
     // them all).  KOKORO_HIP_LSTM_SINGLE=1 selects the one-CU kernel (W_hh partly streamed from L2
     // each step), as does a plan whose pairs or groups gave up before (lstm_single).  Test hook, read
     // at each launch: KOKORO_HIP_TEST_LSTM_SILENT=1 keeps the second half of every pair (the second
-    // part of every group) from publishing and cuts the wait to 10 us, so that they give up.
+    // part of every group; 2: of groups only) from publishing and cuts the wait to 10 us, so that they
+    // give up.
     //   Measured per step: 2.0 us on two CUs, see lstm_split_kernel for the others.
     void recur(const MLstm& l, const float* gx, const int32_t* gx_row, const Dom& d, float* out, int64_t out_ld,
                const std::string& name, int region) {
         static const bool single = env_i64("KOKORO_HIP_LSTM_SINGLE", 0) != 0;
         // KOKORO_HIP_LSTM_QUAD, read at each launch: 1 groups (where they fit the device), 0 pairs for
-        // every span
+        // every span; a context whose recurrences gave up once stays on pairs without it
         check((int)d.len.size() == p->nb, "internal: recurrence domain");
         const int32_t* sched = p->lstm_sched_of(d);
         int64_t longest = 0;
         for (int64_t v : d.len) longest = std::max(longest, v);
-        const int parts = lstm_parts(p->nb, longest, ctx->n_cu, env_i64("KOKORO_HIP_LSTM_QUAD", -1));
-        const bool silent = env_i64("KOKORO_HIP_TEST_LSTM_SILENT", 0) != 0;
+        const int parts = lstm_parts(p->nb, longest, ctx->n_cu, env_i64("KOKORO_HIP_LSTM_QUAD", ctx->lstm_pairs ? 0 : -1));
+        const int64_t hook = env_i64("KOKORO_HIP_TEST_LSTM_SILENT", 0);
+        const bool silent = hook == 1 || (hook == 2 && parts > 2);
         const double v = (double)d.valid();
         label = name;
         launch(PC_LSTM, v * 2 * 1024 * 256 * 2, v * (2048 + 512) * 4 + 2.0 * 1024 * 257 * 4, [&] {
@@ -2306,6 +2310,11 @@ static void check_lstm_abort(kk_plan* p) {
 
 static void run_plan(kk_plan* plan, int until, bool skip_tokens = false);
 
+// A recurrence of the plan gave up: the plan on the one-CU kernel from here, and its context's later
+// batches on pairs (a one-shot call's plan is new with every call: on groups each of them could wait
+// the 2 s out again for as long as the contention lasts).
+static void lstm_gave_up(kk_plan* p) { p->lstm_single = p->ctx->lstm_pairs = true; }
+
 // Drains the stream and reads back the run's abort flag (ids-level plans).
 static bool drain_aborted(kk_plan* p) {
     hipStream_t s = p->ctx->stream;
@@ -2322,7 +2331,7 @@ static bool drain_aborted(kk_plan* p) {
 // and runs again: contention costs time, not an error.  Plans of the other kinds run no recurrence.
 static void drain_and_check_abort(kk_plan* p) {
     if (drain_aborted(p) && !p->lstm_single) {
-        p->lstm_single = true;
+        lstm_gave_up(p);
         run_plan(p, p->last_until);
         drain_aborted(p);
     }
@@ -2423,7 +2432,7 @@ static void init_full_plan(kk_plan* p, const kk_item* items, int n) {
         if (*p->abort_host == 0 || attempt > 0 || p->lstm_single) break;
         // a two-CU pair gave up: the token phase again with the one-CU recurrences (see
         // drain_and_check_abort)
-        p->lstm_single = true;
+        lstm_gave_up(p);
         Runner r{p, ctx, m, ctx->stream};
         r.tokens();
     }
@@ -3247,7 +3256,7 @@ int kk_plan_fetch_wait(kk_plan* plan, char* err, size_t errlen) {
         if (plan->kind == PLAN_FULL && plan->abort_host && *plan->abort_host != 0 && !plan->lstm_single) {
             // a two-CU pair of the run gave up: the run again on the one-CU recurrences (see
             // drain_and_check_abort), its samples into the same destination
-            plan->lstm_single = true;
+            lstm_gave_up(plan);
             run_plan(plan, plan->last_until);
             enqueue_pcm16_fetch(plan, plan->fetch_dst, plan->fetch_clipped);
             drain_aborted(plan);

@@ -10,6 +10,27 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
+def test_context_stays_on_pairs_after_a_give_up():
+    """Groups whose bounded wait runs out (KOKORO_HIP_TEST_LSTM_SILENT=2: a part of every group, but no
+    pair, publishes nothing, 10 us limit) fall back to the one-CU kernel in the call; the context's
+    next calls take pairs, whose results differ from the one-CU kernel's in the last bits."""
+    from kokoro_hip import api, model_spec, workloads
+    items = workloads.small_ids_items(95, [40, 12])
+    ctx = api.Context(0)
+    ctx.upload_model(model_spec.random_model_weights(seed=0))
+    groups = ctx.forward_batch(items)
+    os.environ["KOKORO_HIP_TEST_LSTM_SILENT"] = "2"
+    try:
+        single = ctx.forward_batch(items)
+        after = ctx.forward_batch(items)
+    finally:
+        del os.environ["KOKORO_HIP_TEST_LSTM_SILENT"]
+    assert any(not np.array_equal(a, a2) for (a, _), (a2, _) in zip(single, groups))
+    for (a, d), (a2, d2) in zip(after, groups):
+        assert np.array_equal(d, d2) and np.array_equal(a, a2)
+    ctx.close()
+
+
 @pytest.mark.parametrize("nb", [1, 8, 9, 16, 17, 32, 33])
 def test_split_matches_pair(nb):
     from kokoro_hip import api, model_spec, workloads
