@@ -52,3 +52,26 @@ def test_split_matches_pair(nb):
         for b, ((a, d), (a2, d2)) in enumerate(zip(res[sel], res["0"])):
             assert np.array_equal(d, d2) and np.array_equal(a, a2), (sel, b)
     ctx.close()
+
+
+@pytest.mark.parametrize("nb", [9, 17, 33])
+def test_split_wait_falls_back(nb):
+    """The bounded wait of groups of 8, of 4, and of 4 with lists, forced from the host: the call runs
+    again on the one-CU kernel, so its results are those of pairs that gave up, bit for bit."""
+    from kokoro_hip import api, model_spec, workloads
+    ctx = api.Context(0)
+    ctx.upload_model(model_spec.random_model_weights(seed=0))
+    rng = np.random.default_rng(nb)
+    items = workloads.small_ids_items(97, [int(n) for n in rng.integers(1, 24, nb)])
+    res = {}
+    try:
+        for sel, hook in (("1", "0"), ("1", "2"), ("0", "1")):
+            os.environ["KOKORO_HIP_LSTM_QUAD"], os.environ["KOKORO_HIP_TEST_LSTM_SILENT"] = sel, hook
+            res[sel, hook] = ctx.forward_batch(items)
+    finally:
+        os.environ.pop("KOKORO_HIP_LSTM_QUAD", None)
+        os.environ.pop("KOKORO_HIP_TEST_LSTM_SILENT", None)
+    assert any(not np.array_equal(a, a2) for (a, _), (a2, _) in zip(res["1", "2"], res["1", "0"]))
+    for (a, d), (a2, d2) in zip(res["1", "2"], res["0", "1"]):
+        assert np.array_equal(d, d2) and np.array_equal(a, a2)
+    ctx.close()

@@ -306,9 +306,19 @@ def one_cu_run(full_run, tmp_path_factory):
     return dict(np.load(f))
 
 
-def test_lstm_pair_wait_falls_back_to_one_cu(full_ctx, full_run, one_cu_run):
-    """The two-CU recurrence (this batch's spans are short: the default; KOKORO_HIP_LSTM_QUAD=0 forces
-    it) and its bounded wait, forced from the host: with KOKORO_HIP_TEST_LSTM_SILENT=1 the second
+@pytest.fixture
+def lstm_ctx(full_weights):
+    """A context of the test's own, for tests whose recurrences give up (its later batches take pairs)."""
+    from kokoro_hip import api
+    ctx = api.Context(0)
+    ctx.upload_model(full_weights)
+    yield ctx
+    ctx.close()
+
+
+def test_lstm_pair_wait_falls_back_to_one_cu(lstm_ctx, full_run, one_cu_run):
+    """The two-CU recurrence (KOKORO_HIP_LSTM_QUAD=0 forces it; by default a batch of 3 items runs on 16
+    CUs per sequence) and its bounded wait, forced from the host: with KOKORO_HIP_TEST_LSTM_SILENT=1 the second
     half of every pair publishes nothing and the wait limit is 10 us, so every pair gives up and its
     launch ends.  The call then runs the forward again on the one-CU kernel (which waits on no other
     block) and succeeds: durations and audio bit-identical to a process that used the one-CU kernel
@@ -317,77 +327,83 @@ def test_lstm_pair_wait_falls_back_to_one_cu(full_ctx, full_run, one_cu_run):
     os.environ["KOKORO_HIP_LSTM_QUAD"] = "0"
     os.environ["KOKORO_HIP_TEST_LSTM_SILENT"] = "1"
     try:
-        res = full_ctx.forward_batch(items)
+        res = lstm_ctx.forward_batch(items)
     finally:
         del os.environ["KOKORO_HIP_TEST_LSTM_SILENT"]
         del os.environ["KOKORO_HIP_LSTM_QUAD"]
     for b, (a, d) in enumerate(res):
         assert np.array_equal(d, one_cu_run[f"dur{b}"]) and np.array_equal(a, one_cu_run[f"audio{b}"]), b
-    res = full_ctx.forward_batch(items)
+    res = lstm_ctx.forward_batch(items)
     for (a, d), a2, d2 in zip(res, audio, durs):
         assert np.array_equal(d, d2) and np.array_equal(a, a2)
 
 
-def test_lstm_quad_matches_pair(full_ctx, full_run, one_cu_run):
-    """The four-CU recurrence (KOKORO_HIP_LSTM_QUAD=1 forces it for every span; by default it runs
-    spans of 1,024 steps and more, longer than this batch's): each row's dot product is summed in
-    the two-CU kernel's order, so durations and audio equal the pairs' bit for bit.  Its bounded
-    wait, forced from the host (KOKORO_HIP_TEST_LSTM_SILENT=1: the second quarter of every quad
-    publishes nothing), falls back to the one-CU kernel like the pairs'."""
+def test_lstm_quad_matches_pair(lstm_ctx, full_run, one_cu_run):
+    """The recurrence on 16 CUs per sequence (this batch's default; KOKORO_HIP_LSTM_QUAD=1 forces groups
+    for every span): each row's dot product is summed in the two-CU kernel's order, so durations and
+    audio equal the pairs' (KOKORO_HIP_LSTM_QUAD=0) bit for bit.  Its bounded wait, forced from the
+    host (KOKORO_HIP_TEST_LSTM_SILENT=1: the second part of every group publishes nothing), falls
+    back to the one-CU kernel like the pairs'."""
     items, audio, durs, _ = full_run
-    os.environ["KOKORO_HIP_LSTM_QUAD"] = "1"
+    res = {}
     try:
-        res = full_ctx.forward_batch(items)
-        for b, ((a, d), a2, d2) in enumerate(zip(res, audio, durs)):
+        for sel in ("0", "1"):
+            os.environ["KOKORO_HIP_LSTM_QUAD"] = sel
+            res[sel] = lstm_ctx.forward_batch(items)
+        for b, ((a, d), (a2, d2)) in enumerate(zip(res["1"], res["0"])):
             assert np.array_equal(d, d2) and np.array_equal(a, a2), b
+            assert np.array_equal(d, durs[b]) and np.array_equal(a, audio[b]), b
         os.environ["KOKORO_HIP_TEST_LSTM_SILENT"] = "1"
         try:
-            res = full_ctx.forward_batch(items)
+            res = lstm_ctx.forward_batch(items)
         finally:
             del os.environ["KOKORO_HIP_TEST_LSTM_SILENT"]
         for b, (a, d) in enumerate(res):
             assert np.array_equal(d, one_cu_run[f"dur{b}"]) and np.array_equal(a, one_cu_run[f"audio{b}"]), b
     finally:
         del os.environ["KOKORO_HIP_LSTM_QUAD"]
-    res = full_ctx.forward_batch(items)
+    res = lstm_ctx.forward_batch(items)
     for (a, d), a2, d2 in zip(res, audio, durs):
         assert np.array_equal(d, d2) and np.array_equal(a, a2)
 
 
 def test_lstm_quad_lists_match_pairs(full_ctx):
-    """More sequences than quads: 40 items are 80 sequences on 64 quads, so 16 quads run two
-    sequences one after another (the schedule gives the short ones to the quads that finish first)
+    """More sequences than groups: 40 items are 80 sequences on 64 groups of 4, so 16 groups run two
+    sequences one after another (the schedule gives the short ones to the groups that finish first)
     -- some of them in the other direction, with the W_hh rows reloaded.  Durations and audio equal
     the two-CU kernel's (every sequence on its own pair) bit for bit."""
     from kokoro_hip import workloads
     rng = np.random.default_rng(46)
     items = workloads.small_ids_items(46, [int(n) for n in rng.integers(3, 40, 40)])
     res = {}
-    for sel in ("1", "0"):  # quads, pairs
+    for sel in ("1", "0"):  # groups, pairs
         os.environ["KOKORO_HIP_LSTM_QUAD"] = sel
         try:
             res[sel] = full_ctx.forward_batch(items)
         finally:
             del os.environ["KOKORO_HIP_LSTM_QUAD"]
-    quads, pairs = res["1"], res["0"]
-    for b, ((a, d), (a2, d2)) in enumerate(zip(quads, pairs)):
+    groups, pairs = res["1"], res["0"]
+    for b, ((a, d), (a2, d2)) in enumerate(zip(groups, pairs)):
         assert np.array_equal(d, d2) and np.array_equal(a, a2), b
 
 
-def test_lstm_abort_falls_back_in_every_result_path(full_ctx, full_run, one_cu_run):
+@pytest.mark.parametrize("sel", ["0", "1"])  # pairs, groups of 16
+def test_lstm_abort_falls_back_in_every_result_path(lstm_ctx, full_run, one_cu_run, monkeypatch, sel):
     """A plan run whose recurrences give up (KOKORO_HIP_TEST_LSTM_SILENT=1, read at each run) would
     leave h rows of an earlier run behind; every path that hands results back -- sync, fetch,
     fetch_pcm16, the asynchronous fetch's wait, taps -- runs the plan again on the one-CU kernel
-    first, and returns that run's results.  Per path, a plan created on the pairs, run with the hook:
+    first, and returns that run's results.  Per path, a plan created on pairs or groups, run with the
+    hook:
     - the call succeeds; t_en (the text encoder: ids only) equals the one-CU process's bit for bit;
     - the plan stays on the one-CU kernel: a further run gives the same audio, PCM_16 equal to
       fetch_pcm16 of that audio."""
     from kokoro_hip import api
     items, _, durs, _ = full_run
     T0 = len(items[0].ids)
+    monkeypatch.setenv("KOKORO_HIP_LSTM_QUAD", sel)
 
     def plan_after_silent_run():
-        plan = api.Plan.full(full_ctx, items)
+        plan = api.Plan.full(lstm_ctx, items)
         os.environ["KOKORO_HIP_TEST_LSTM_SILENT"] = "1"
         try:
             plan.run()
@@ -396,7 +412,7 @@ def test_lstm_abort_falls_back_in_every_result_path(full_ctx, full_run, one_cu_r
         return plan
 
     def pcm_async(plan):
-        pcm = api.PinnedArray(full_ctx, 600 * sum(int(d.sum()) + 2 for d in plan.durations), np.int16)
+        pcm = api.PinnedArray(lstm_ctx, 600 * sum(int(d.sum()) + 2 for d in plan.durations), np.int16)
         try:
             plan.fetch_pcm16_async(pcm)
             plan.fetch_wait()
@@ -426,8 +442,8 @@ def test_lstm_abort_falls_back_in_every_result_path(full_ctx, full_run, one_cu_r
 
 
 def test_lstm_pair_matches_one_cu_kernel(full_run, one_cu_run):
-    """The two-CU recurrence against the one-CU kernel on the same batch: the same arithmetic in
-    another summation order.
+    """The recurrence on several CUs (the pairs' sums, bit for bit, also on this batch's 16) against the
+    one-CU kernel on the same batch: the same arithmetic in another summation order.
     - t_en: the text encoder's recurrence on identical inputs (its conv stack does not depend on the
       switch), so the outputs differ by f32 rounding only: >= 120 dB;
     - d, logits, shared: chains of recurrences joined by linear layers with bf16-rounded operands,
@@ -448,7 +464,7 @@ def test_lstm_pair_matches_one_cu_kernel(full_run, one_cu_run):
             if name == "shared" and not same:
                 continue  # another frame count
             snr = snr_db(one[f"{name}{b}"], taps[b][name])
-            _print(f"  item {b} {name}: pair vs one-CU kernel {snr:.1f} dB")
+            _print(f"  item {b} {name}: 16 CUs vs one-CU kernel {snr:.1f} dB")
             assert snr >= bar, (b, name)
 
 
