@@ -1819,6 +1819,19 @@ struct Runner {
         launch(PC_SOURCE, 0, n2 * 4 * (1 + kHarmonics) + nfr120 * 88, [&] { return launch_source_stft(q, s); });
     }
 
+    // How many stages' noise branches go before the decoder's launches (their convolutions and
+    // statistics are ~25 launches; enqueued first they keep the main stream idle for ~110 us, enqueued
+    // last the generator's stage 0 waits for its own).  Decoder calls, both stages first = 1 (calls from ids
+    // do not change by more than 0.4%, the recurrences come before):
+    //   none first: 40 frames 0.91, 405 0.95; of more than 8 items up to 2,048 frames 0.93 to 0.99; of few
+    //     items 1.02 to 1.05 at 430, 1.02 at 480 to 650 and 1.02 at 1,100 frames, 0.98 to 0.99 from 1,300;
+    //   stage 0's first: 0.95 at 40 and 0.97 at 405 frames; few items 0.95 to 0.99 at 430 to 1,200, 0.99 at
+    //     1,300 to 2,000; 0.98 to 0.99 with 16 to 30 items;
+    //   past 2,048 frames the host is ahead: 0.99 to 1.01 for either.
+    static int noise_stages_early(int64_t frames, int items) {
+        if (frames > 2048) return 2;
+        return frames > 409 && frames <= 1200 && items <= 8 ? 1 : 0;  // (up to 409: stage 0 in grouped launches)
+    }
     // xs_i = noise_res[i](noise_convs[i](masked spec)) (src/gpu_batch.rs:362-375) into p->xs[i],
     // with its own h, statistics region (3) and coefficient pair, so that it can run beside the
     // decoder and the previous stage.
@@ -2244,25 +2257,24 @@ struct Runner {
             noise_conv(0);
             s = main_s;
         }
-        auto noise_rest = [&]() {
+        // stages [from, to)'s noise branches (stage 0's conv is enqueued above)
+        auto noise = [&](int from, int to) {
+            if (!conc) return;
             s = ctx->side[2];
-            noise_resblock(0);
-            KK_HIP(hipEventRecord(p->noise_ev[1], s));
-            if (until > KK_STAGE_GEN0) {
-                noise_branch(1);
-                KK_HIP(hipEventRecord(p->noise_ev[2], s));
+            for (int i = from; i < to && (i == 0 || until > KK_STAGE_GEN0); i++) {
+                if (i == 0)
+                    noise_resblock(0);
+                else
+                    noise_branch(1);
+                KK_HIP(hipEventRecord(p->noise_ev[1 + i], s));
             }
             s = main_s;
         };
-        // Short calls: the decoder's launches before the rest of the noise branches', whose 25 launches
-        // kept the main stream idle for ~110 us (of 900 on a 40-frame item).  Calls of more frames
-        // are not bound by the host and fill the GPU with the noise branches while t_en is staged
-        // (13,501 frames: 0.3 to 1% slower the other way round).
-        const bool decoder_first = frames() <= 2048;
-        if (conc && !decoder_first) noise_rest();
+        const int early = noise_stages_early(frames(), p->nb);
+        noise(0, early);
         if (p->late_items && !dry) stage_late_ten();
         if (p->kind == PLAN_DECODER || p->kind == PLAN_FULL) decoder();
-        if (conc && decoder_first) noise_rest();
+        noise(early, 2);
         if (until <= KK_STAGE_DECODER) return;
         if (!conc) source();
         if (until <= KK_STAGE_SOURCE) return;
