@@ -11,7 +11,7 @@
  * Threading: a context may be created on one thread and used from another (the reference creates
  * its Gpu on a helper thread, src/engine.rs:92-96); every entry selects the context's device
  * itself.  Calls on one context must not overlap (the reference engine is not shared,
- * src/cli.rs:625-626).
+ * src/cli.rs:625-626), except those of kk_encode_pcm16 with each other.
  */
 #ifndef KOKORO_HIP_H
 #define KOKORO_HIP_H
@@ -303,7 +303,10 @@ void kk_host_free(void* p);
 int kk_plan_item_samples(const kk_plan* plan, int item, int64_t* offset, int64_t* count);
 int kk_plan_fetch_pcm16_async(kk_plan* plan, int16_t* dst, int64_t* clipped, char* err, size_t errlen);
 int kk_plan_fetch_wait(kk_plan* plan, char* err, size_t errlen);
-/* The same encoding of a host array (uploads, encodes on the device, downloads). */
+/* The same encoding of a host array (uploads, encodes on the device, downloads).  The context keeps
+ * the device buffer between calls (at most 16 MiB: 2.79 million samples); a longer call, and one that
+ * finds it in use by a call on another thread, allocates its own and frees it.  A failure of a one-shot
+ * entry (kk_forward_batch, kk_forward_decoder_batch) releases it. */
 int kk_encode_pcm16(kk_ctx* ctx, const float* audio, int64_t n, int16_t* out, int64_t* clipped, char* err,
                     size_t errlen);
 /* The canonical 44-byte mono RIFF/WAVE header (wav::header, src/wav.rs:43-61): format tag 1

@@ -2556,6 +2556,15 @@ static void drop_oneshot(kk_ctx* ctx) {
     ctx->oneshot = nullptr;
 }
 
+// Everything the context keeps between calls: after a failure of a one-shot entry (device memory
+// exhausted above all), so that a caller splitting the batch (src/engine.rs:229-234) has the whole
+// device again.  (A kk_encode_pcm16 buffer in use by a call on another thread stays.)
+static void release_kept(kk_ctx* ctx) {
+    drop_oneshot(ctx);
+    std::unique_lock<std::mutex> lk(ctx->pcm_mu, std::try_to_lock);
+    if (lk.owns_lock()) ctx->pcm_buf.release();
+}
+
 // ------------------------------------------------------------------ host output memory
 // The audio of kk_plan_fetch / kk_forward_decoder_batch lands in pinned host blocks that the
 // library keeps for reuse: one block per fetch holds the whole packed sample layout (one DMA copy,
@@ -3277,7 +3286,7 @@ int kk_plan_fetch_wait(kk_plan* plan, char* err, size_t errlen) {
     });
 }
 
-// 2.6 million samples: 116 s of audio.
+// 2.79 million samples of 4 + 2 bytes: 116 s of audio at 24 kHz.
 static constexpr size_t kPcmKeepBytes = 16 << 20;
 
 int kk_encode_pcm16(kk_ctx* ctx, const float* audio, int64_t n, int16_t* out, int64_t* clipped, char* err,
@@ -3478,9 +3487,7 @@ int kk_forward_decoder_batch(kk_ctx* ctx, const kk_decoder_item* items, int n, k
                              ms(t2, t3), ms(t3, t4));
             }
         } catch (...) {
-            // a failure (device memory exhausted above all) releases the cached buffers, so that a
-            // caller splitting the batch (src/engine.rs:229-234) has the whole device again
-            drop_oneshot(ctx);
+            release_kept(ctx);
             throw;
         }
     });
@@ -3524,7 +3531,7 @@ int kk_forward_batch(kk_ctx* ctx, const kk_item* items, int n, kk_result* out, c
                              ms(t0, t1), ms(t1, t2), ms(t2, t3));
             }
         } catch (...) {
-            drop_oneshot(ctx);
+            release_kept(ctx);
             throw;
         }
     });

@@ -1,5 +1,7 @@
 """kk_encode_pcm16 keeps its device buffer between calls up to a bound: calls of other lengths before
-and after, beyond the bound, and from two threads at once encode as the oracle does."""
+and after, beyond the bound, and from two threads at once encode as the oracle does; a one-shot call
+that fails gives it back."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -37,3 +39,32 @@ def test_two_threads(gpu_ctx):
     for t in ts:
         t.join()
     assert ok == [True, True]
+
+
+def test_failed_one_shot_call_releases_the_buffer(gpu_ctx, monkeypatch):
+    """A caller that splits its batch after KK_ERR_OOM has the whole device: no 16 MB stay behind."""
+    from kokoro_hip import api, workloads
+    hip = C.CDLL("libamdhip64.so.7")  # the runtime that the library is bound to
+    hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+    items = workloads.small_items(5, [3])
+
+    def fail():
+        with pytest.raises(api.KKError) as e:
+            gpu_ctx.forward_decoder_batch(items)
+        assert e.value.code == -3
+
+    def free():
+        f, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(total)) == 0
+        return f.value
+
+    monkeypatch.setenv("KOKORO_HIP_TEST_OOM_ABOVE", "0")
+    fail()  # what earlier calls kept
+    before = free()
+    a = wave(2_700_000, 3)  # 16.2 MB
+    assert same(gpu_ctx, a)
+    kept = free()
+    assert before - kept >= 16_000_000
+    fail()
+    assert free() - kept >= 16_000_000
+    assert same(gpu_ctx, a)
