@@ -562,7 +562,7 @@ __global__ __launch_bounds__(64 * WM * WN + kNP) void conv_mfma_kernel(ConvParam
     constexpr bool CONVT = EPI == EPI_CONVT || EPI == EPI_CONVT_REFLECT;
     float* bias_s = (float*)(xs + 2 * slab_elems) + NC / 64 * 32 * kScrLd;
     if constexpr (!CONVT) {
-        for (int i = threadIdx.x; i < p.m_pad; i += NC) bias_s[i] = i < p.m ? p.bias[i] : 0.f;
+        for (int i = threadIdx.x; i < p.m_pad; i += NC) bias_s[i] = row_bias(p.bias, i, p.m);
     }
     f32x16 acc[MI][4];
 

@@ -201,8 +201,7 @@ __global__ __launch_bounds__(128 * WM + kNP) void conv_narrow_kernel(ConvGroup g
         for (int g = 0; g < 4; g++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                // (rows past the layer's are computed and not stored)
-                const float bv = CONVT ? 0.f : p.bias[min(u.m0 + wm * 32 + 8 * g + 4 * lh + e, p.m - 1)];
+                const float bv = CONVT ? 0.f : row_bias(p.bias, u.m0 + wm * 32 + 8 * g + 4 * lh + e, p.m);
 #pragma unroll
                 for (int j = 0; j < NJ; j++) acc[j][4 * g + e] = bv;
             }
@@ -452,8 +451,6 @@ hipError_t launch_narrow_t(const ConvGroup& g, int64_t blocks, int max_halo, int
 }  // namespace
 
 hipError_t launch_conv_narrow(ConvGroup& g, int pro, int epi, bool stats, bool in_h, bool out_h, hipStream_t s) {
-    int64_t blocks = 0;
-    int max_halo = 0;
     // The smallest blocks that leave the launch at most one block per CU: 64 columns without
     // statistics, then 32 rows while they fill at most half of the CUs (a block's K loop is bound by
     // its own waves: 32 rows take 0.18 us per tap of 64 channels where 64 rows take 0.21; past 128
@@ -462,7 +459,8 @@ hipError_t launch_conv_narrow(ConvGroup& g, int pro, int epi, bool stats, bool i
     for (int i = 0; i < g.n; i++) units += conv_units64(g.p[i]);
     const int bn = stats || 2 * units > 256 ? 128 : 64;
     const int bm = units * (128 / bn) * 2 <= 128 ? 32 : 64;
-    blocks = 0;
+    int64_t blocks = 0;
+    int max_halo = 0;
     for (int i = 0; i < g.n; i++) {
         const ConvParams& p = g.p[i];
         const bool convt = epi == EPI_CONVT || epi == EPI_CONVT_REFLECT;

@@ -56,6 +56,13 @@ inline int64_t walk_grid(int64_t count, int mblocks, int n_cu) {
     return units < fit ? units : fit;
 }
 
+// What an accumulator of output row r starts at: the bias, 0 past the layer's m rows (their weights are 0
+// too, and stores of four rows at a time reach up to three of them).
+__host__ __device__ inline float row_bias(const float* bias, int r, int m) {
+    const float b = bias[r < m ? r : m - 1];
+    return r < m ? b : 0.f;
+}
+
 // A ConvT unit's columns (EPI_CONVT / EPI_CONVT_REFLECT): tile column col (of nv valid, from input
 // column n0) is output row o = stride (n0 + col) + ph - pad, written -- as row o, or o + 1 with the
 // reflection pad -- when o lies in the item's output span [os, os + ol) (ol without the reflected

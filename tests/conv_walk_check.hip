@@ -148,12 +148,25 @@ static long check_convt_cols() {
     return bad;
 }
 
+// A row's starting value: its bias, and 0 past the layer's rows, without a read past the bias.
+static long check_row_bias() {
+    long bad = 0;
+    for (int m : {1, 22, 50, 63, 64}) {
+        std::vector<float> bias(m);
+        for (int r = 0; r < m; r++) bias[r] = 1.f + r;
+        for (int r = 0; r < 128; r++)
+            if (kk::row_bias(bias.data(), r, m) != (r < m ? 1.f + r : 0.f)) bad++;
+    }
+    return bad;
+}
+
 int main(int argc, char** argv) {
     plant = argc > 1 && std::strcmp(argv[1], "--plant") == 0;
     if (!plant) {
         const long bc = check_convt_cols();
         std::printf("convt columns violations %ld\n", bc);
         if (bc) return 1;
+        std::printf("row bias violations %ld\n", check_row_bias());
     }
     const int64_t counts[] = {1, 2, 7, 8, 9, 17, 64, 257, 1000};
     const int mbs[] = {1, 2, 3, 4};
