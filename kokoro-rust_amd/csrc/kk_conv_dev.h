@@ -19,7 +19,7 @@ constexpr int kRS = kCK + 8;  // LDS row stride (bf16 elements, 144 bytes)
 constexpr int kNJ = 8;        // 16-column MFMA tiles per wave (wave N = 128)
 constexpr int kMaxHalo = 64;    // largest (k - 1) * dil the staging covers
 constexpr int kSmallHalo = 16;  // layers with (k - 1) * dil up to this run fewer producer passes
-constexpr int kNP = 256;      // producer threads per block (kk_conv.hip)
+constexpr int kNP = 256;      // producer threads per block
 
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -77,9 +77,9 @@ __device__ __forceinline__ float vgpr_f(float x) { return __int_as_float(vgpr(__
 // number of loads is fixed and the producers' wait counts are static), convert() applies the
 // prologue and writes bf16 rows into an LDS buffer.  Rows outside the item, and channels >= cin,
 // are staged as 0 (the conv's zero padding of the activated signal).
-template <int PRO, bool IN_H, int BN, int MAXH, int NP = kNP>
+template <int PRO, bool IN_H, int BN, int MAXH>
 struct Slot {
-    static constexpr int RP = NP / 16;                    // rows per pass
+    static constexpr int RP = kNP / 16;                   // rows per pass
     static constexpr int RB = (BN + MAXH + RP - 1) / RP;  // passes (MAXH: the largest halo served)
     static constexpr bool WIDE = PRO != PRO_BF16 && !IN_H;    // f32 source: 4 dwords per quad
     static constexpr int NW = WIDE ? 4 : 2;

@@ -747,7 +747,7 @@ struct kk_plan {
     kk::Dom dn, d2, d20, d120, ds;
     // test hooks read at plan creation (see apply_test_hooks)
     bool nomask = false, poison = false, tap_source = false;
-    // the recurrences on the one-CU kernel: set once a two-CU pair of this plan gave up (the plan's
+    // the recurrences on the one-CU kernel: set once a recurrence of this plan gave up (the plan's
     // later runs stay there), reset for each new batch
     bool lstm_single = false;
     // snake plans
@@ -2228,7 +2228,7 @@ struct Runner {
             prosody();
             if (until <= KK_STAGE_PROSODY) return;
         }
-        // a Snake block's plan: only the rows of its own AdaINs (a few hundred of the table's 37,504)
+        // a Snake block's plan: only the rows of its own AdaINs (1,536 or 3,072 of the table's 37,396)
         int row0 = 0, row1 = m.style_rows;
         if (p->kind == PLAN_SNAKE) {
             row0 = m.style_rows, row1 = 0;
@@ -2307,16 +2307,11 @@ static void prebuild_tiles(kk_plan* p) {
     r.run(KK_STAGE_ALL);
 }
 
-// Fills plan p (new, or the one-shot plan whose device buffers are reused) for an ids-level batch
-// (GpuKokoro::forward_batch, src/gpu_batch.rs:179-297).  Phase A, at once: the token layout
-// (src/gpu_batch.rs:188-197), the token phase on the device, its logits back to the host and the
-// durations (src/gpu_batch.rs:234-248).  Phase B: the frame layout and everything after, as a
-// decoder plan whose t_en, F0 and N the plan computes itself.
-// A two-CU recurrence whose block waited more than 2 s for its partner ends every block of its
+// A recurrence whose block waited more than 2 s for its partners ends every block of its
 // launch and leaves the run's abort flag set (read back into abort_host with the run's last copy).
 static void check_lstm_abort(kk_plan* p) {
     if (p->abort_host && *p->abort_host != 0)
-        fail(KK_ERR_HIP, "BiLSTM recurrence: a block of a two-CU pair waited more than 2 s for its partner "
+        fail(KK_ERR_HIP, "BiLSTM recurrence: a block waited more than 2 s for the sequence's other blocks "
                           "(set KOKORO_HIP_LSTM_SINGLE=1 for the one-CU kernel)");
 }
 
@@ -2338,7 +2333,7 @@ static bool drain_aborted(kk_plan* p) {
 
 // Every path that hands an ids-level plan's results to the caller (audio, PCM, taps, sync) drains the
 // stream and checks that no recurrence of the last run gave up (its h rows would hold an earlier
-// run's values).  If one did -- a two-CU pair whose partner was held off its CU past the 2 s bound,
+// run's values).  If one did -- a block held off its CU past the 2 s bound that its partners wait,
 // e.g. by another process -- the plan switches to the one-CU kernel, which waits on no other block,
 // and runs again: contention costs time, not an error.  Plans of the other kinds run no recurrence.
 static void drain_and_check_abort(kk_plan* p) {
@@ -2350,7 +2345,11 @@ static void drain_and_check_abort(kk_plan* p) {
     if (p->kind == PLAN_FULL) check_lstm_abort(p);
 }
 
-
+// Fills plan p (new, or the one-shot plan whose device buffers are reused) for an ids-level batch
+// (GpuKokoro::forward_batch, src/gpu_batch.rs:179-297).  Phase A, at once: the token layout
+// (src/gpu_batch.rs:188-197), the token phase on the device, its logits back to the host and the
+// durations (src/gpu_batch.rs:234-248).  Phase B: the frame layout and everything after, as a
+// decoder plan whose t_en, F0 and N the plan computes itself.
 static void init_full_plan(kk_plan* p, const kk_item* items, int n) {
     kk_ctx* ctx = p->ctx;
     const Model& m = ctx->model;
@@ -2442,7 +2441,7 @@ static void init_full_plan(kk_plan* p, const kk_item* items, int n) {
         KK_HIP(hipMemcpyAsync(p->abort_host, p->u_lstmx.p, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
         KK_HIP(hipStreamSynchronize(ctx->stream));
         if (*p->abort_host == 0 || attempt > 0 || p->lstm_single) break;
-        // a two-CU pair gave up: the token phase again with the one-CU recurrences (see
+        // a recurrence gave up: the token phase again with the one-CU recurrences (see
         // drain_and_check_abort)
         lstm_gave_up(p);
         Runner r{p, ctx, m, ctx->stream};
@@ -3275,7 +3274,7 @@ int kk_plan_fetch_wait(kk_plan* plan, char* err, size_t errlen) {
         plan->fetch_pending = false;
         KK_HIP(hipEventSynchronize(plan->fetch_ev));
         if (plan->kind == PLAN_FULL && plan->abort_host && *plan->abort_host != 0 && !plan->lstm_single) {
-            // a two-CU pair of the run gave up: the run again on the one-CU recurrences (see
+            // a recurrence of the run gave up: the run again on the one-CU recurrences (see
             // drain_and_check_abort), its samples into the same destination
             lstm_gave_up(plan);
             run_plan(plan, plan->last_until);

@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256 * T) void stats_fin_kernel(const float* __restr
 // in f64.  W is stored transposed [128][ld] so consecutive threads read consecutive rows.  A block
 // covers 64 rows; its four waves take one quarter of k each (the loads of a quarter issued
 // together), and the quarters' sums meet in LDS, E items per pass.  Bound by the table's read (the
-// decoder's and generator's 37,504 rows: 19 MB) and, from a few items on, by the f64 sums: E is the
+// decoder's and generator's 37,396 rows: 19 MB) and, from a few items on, by the f64 sums: E is the
 // smallest of 1, 4 and 16 that holds the batch, as sums of items that are not there cost as much as
 // real ones.  Of few rows (kStyleFewRows; one Snake block's AdaINs) the passes run in blocks of 4
 // items each beside each other, reading the rows again from the L2.  Measured

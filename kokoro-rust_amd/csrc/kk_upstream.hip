@@ -587,6 +587,21 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_pair_kernel(const float* gx
     }
 }
 
+// acc += w[k + i][e] h[i] for i = 0 .. 15 in sequence, h[i] in lane i of each row of 16 lanes of h: one
+// v_fmac_f32 with a DPP operand each (the compiler makes a move and a multiply-add of it).  The s_nop
+// covers the two wait states between a VALU write of h and its DPP read.
+template <int RPT>
+__device__ __forceinline__ void fma16(float& acc, float h, const float (&w)[64][RPT], int k, int e) {
+#define KK_FM(i, op) "v_fmac_f32_dpp %0, %1, %" #op " row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" KK_FM(0, 2) KK_FM(1, 3) KK_FM(2, 4) KK_FM(3, 5) KK_FM(4, 6) KK_FM(5, 7) KK_FM(6, 8) KK_FM(7, 9)
+            KK_FM(8, 10) KK_FM(9, 11) KK_FM(10, 12) KK_FM(11, 13) KK_FM(12, 14) KK_FM(13, 15) KK_FM(14, 16) KK_FM(15, 17)
+        : "+v"(acc)
+        : "v"(h), "v"(w[k][e]), "v"(w[k + 1][e]), "v"(w[k + 2][e]), "v"(w[k + 3][e]), "v"(w[k + 4][e]), "v"(w[k + 5][e]),
+          "v"(w[k + 6][e]), "v"(w[k + 7][e]), "v"(w[k + 8][e]), "v"(w[k + 9][e]), "v"(w[k + 10][e]), "v"(w[k + 11][e]),
+          "v"(w[k + 12][e]), "v"(w[k + 13][e]), "v"(w[k + 14][e]), "v"(w[k + 15][e]));
+#undef KK_FM
+}
+
 // The BiLSTM recurrence on P = 4, 8 or 16 CUs per (item, direction): block part pt owns the U = 256 / P
 // hidden units [U pt, U pt + U), i.e. 4 U gate rows, and keeps all of their W_hh in registers (each
 // thread RPT gate rows over one 64-long k-quarter).  Each step a block computes its U units of h and
@@ -609,29 +624,13 @@ __global__ void __launch_bounds__(kLstmThreads) lstm_pair_kernel(const float* gx
 // groups that finish first.  A group reloads its W_hh rows only when the direction changes; every
 // sequence starts from h = c = 0 and has its own exchange words.  A block whose partners are not
 // resident yet waits for slots that finishing groups release; kk_lstm.h says which P leave a slot for
-// them whatever runs beside this launch.  Every wait is bounded as in the pair kernel.
+// them beside the process's other launches.  Every wait is bounded as in the pair kernel.
 //   sched: [nq + 1] list offsets, then the sequence ids (2 item + direction) of the groups' lists.
-// acc += w[k + i][e] h[i] for i = 0 .. 15 in sequence, h[i] in lane i of each row of 16 lanes of h: one
-// v_fmac_f32 with a DPP operand each (the compiler makes a move and a multiply-add of it).  The s_nop
-// covers the two wait states between a VALU write of h and its DPP read.
-template <int RPT>
-__device__ __forceinline__ void fma16(float& acc, float h, const float (&w)[64][RPT], int k, int e) {
-#define KK_FM(i, op) "v_fmac_f32_dpp %0, %1, %" #op " row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n\t"
-    asm("s_nop 1\n\t" KK_FM(0, 2) KK_FM(1, 3) KK_FM(2, 4) KK_FM(3, 5) KK_FM(4, 6) KK_FM(5, 7) KK_FM(6, 8) KK_FM(7, 9)
-            KK_FM(8, 10) KK_FM(9, 11) KK_FM(10, 12) KK_FM(11, 13) KK_FM(12, 14) KK_FM(13, 15) KK_FM(14, 16) KK_FM(15, 17)
-        : "+v"(acc)
-        : "v"(h), "v"(w[k][e]), "v"(w[k + 1][e]), "v"(w[k + 2][e]), "v"(w[k + 3][e]), "v"(w[k + 4][e]), "v"(w[k + 5][e]),
-          "v"(w[k + 6][e]), "v"(w[k + 7][e]), "v"(w[k + 8][e]), "v"(w[k + 9][e]), "v"(w[k + 10][e]), "v"(w[k + 11][e]),
-          "v"(w[k + 12][e]), "v"(w[k + 13][e]), "v"(w[k + 14][e]), "v"(w[k + 15][e]));
-#undef KK_FM
-}
 template <int P>  // (two blocks per CU at P = 8 and 16: 4 waves per SIMD; lstm_blocks_per_cu counts on it)
-__global__ void __launch_bounds__(kLstmThreads, 2 * lstm_blocks_per_cu(P)) lstm_split_kernel(const float* gx, int64_t gx_ld, const int32_t* gx_row,
-                                                                  const int64_t* start, const int64_t* len,
-                                                                  const int32_t* sched, int nq, const float* whh_t,
-                                                                  const float* bhh, float* out, int64_t out_ld,
-                                                                  uint64_t* xbuf, int* abort, uint64_t wait_ticks,
-                                                                  int silent_part) {
+__global__ void __launch_bounds__(kLstmThreads, 2 * lstm_blocks_per_cu(P))
+lstm_split_kernel(const float* gx, int64_t gx_ld, const int32_t* gx_row, const int64_t* start, const int64_t* len,
+                  const int32_t* sched, int nq, const float* whh_t, const float* bhh, float* out, int64_t out_ld,
+                  uint64_t* xbuf, int* abort, uint64_t wait_ticks, int silent_part) {
     constexpr int U = kH / P, R = 4 * U;      // this block's units and gate rows
     constexpr int RPT = P == 4 ? 2 : 1;       // gate rows per thread
     constexpr int NQT = R / RPT;              // threads per k-quarter
