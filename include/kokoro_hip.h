@@ -318,7 +318,10 @@ int kk_wav_header(int format, uint32_t sample_rate, uint64_t data_bytes, uint8_t
 
 /* ------------------------------------------------------------------ measurement
  * With profiling on, kk_plan_run runs every kernel on the context's stream (no side streams, so
- * each kernel has the GPU to itself) and brackets every launch with HIP events there;
+ * each kernel has the GPU to itself), every layer in a launch of its own, and brackets every launch
+ * with HIP events there.  An unprofiled run of few units puts up to three layers (and their AdaINs)
+ * into one launch and a standalone statistics pass with its coefficients into another, so its launches
+ * are fewer than the ones reported here (same results, bit for bit).
  * kk_profile_read reports, per kernel class with at least one launch since the last read, the summed
  * event time and the algorithmic FLOP and bytes of those launches (valid rows only; bytes = the
  * data the step must read and write once).  Classes: the MFMA convolutions "snake_conv",
